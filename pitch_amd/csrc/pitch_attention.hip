@@ -22,7 +22,7 @@
 // Query heads of one KV head (grouped-query attention) share every table read; their count is padded to
 // 1, 2, 4 or 8 (padded queries are zero and never written out). With 4 or 8 the scores' and the values' products
 // run on the matrix cores (v_mfma_f32_4x4x1f32, below).
-#include "pitch_device.h"
+#include "pitch_attn_shared.h"
 
 #ifndef PITCH_DIM
 #error "compile with -DPITCH_DIM=<dim>"
@@ -38,7 +38,6 @@ constexpr int kMaxChunk = 1024;          // tokens per workgroup; a chunk's scor
 #ifndef PITCH_ATTN_MFMA
 #define PITCH_ATTN_MFMA 1  // four or eight query heads: their products on the matrix cores (below)
 #endif
-constexpr float kLn2 = 0x1.62e430p-1f;   // ln(2)
 
 // Matrix-core products for four or eight query heads per KV head. v_mfma_f32_4x4x1f32 computes 16 independent
 // 4 x 4 outer products per wave: D[v] of lane l += A(lane 4 (l / 4) + v) * B(lane l), in float32 (lane layout
@@ -877,19 +876,13 @@ __global__ __launch_bounds__(kBlock) void attn_combine(AttnArgs a) {
   __shared__ float s_part[4 * (D + 1)];
   const uint32_t kv = blockIdx.x / a.nq, h = blockIdx.x % a.nq;
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-  const WsLayout L(a);
-  const float* ml = a.ws + L.ml + ((uint64_t)kv * a.nqp + h) * a.chunks * 2;
-  const float* A = a.ws + L.acc + ((uint64_t)kv * a.nqp + h) * a.chunks * D;
-  float M = -__builtin_inff();
-  for (uint32_t c = tid; c < a.chunks; c += kBlock) M = fmaxf(M, ml[2 * c]);
-  for (int off = 1; off < 64; off <<= 1) M = fmaxf(M, __shfl_xor(M, off));
-  if (lane == 0) s_red[wid] = M;
-  __syncthreads();
-  M = fmaxf(fmaxf(s_red[0], s_red[1]), fmaxf(s_red[2], s_red[3]));
-  float ls = 0.f, acc[E];
+  const float* ml = a.ws + a.ws_ml + ((uint64_t)kv * a.nqp + h) * a.chunks * 2;
+  const float* A = a.ws + a.ws_acc + ((uint64_t)kv * a.nqp + h) * a.chunks * D;
+  // wave w merges chunks w, w + 4, ... as it reads them (maxima, sums and accumulators in one round of loads, kU chunks
+  // at a time), then the waves merge through LDS
+  float M = -__builtin_inff(), ls = 0.f, acc[E];
 #pragma unroll
   for (int e = 0; e < E; ++e) acc[e] = 0.f;
-  // chunks c = wid, wid + 4, ...; loads are issued kU chunks at a time so they overlap
   constexpr int kU = 16;
   for (uint32_t c0 = wid; c0 < a.chunks; c0 += 4 * kU) {
     float mv[kU], lv[kU], av[kU][E];
@@ -903,6 +896,14 @@ __global__ __launch_bounds__(kBlock) void attn_combine(AttnArgs a) {
 #pragma unroll
       for (int e = 0; e < E; ++e) av[u][e] = A[(uint64_t)cc * D + lane * E + e];
     }
+    float m = M;
+#pragma unroll
+    for (int u = 0; u < kU; ++u) m = fmaxf(m, mv[u]);
+    const float g = M == m ? 1.f : exp2f(M - m);
+    M = m;
+    ls *= g;
+#pragma unroll
+    for (int e = 0; e < E; ++e) acc[e] *= g;
 #pragma unroll
     for (int u = 0; u < kU; ++u) {
       const float f = exp2f(mv[u] - M);  // 0 for chunks past the end
@@ -913,16 +914,26 @@ __global__ __launch_bounds__(kBlock) void attn_combine(AttnArgs a) {
   }
 #pragma unroll
   for (int e = 0; e < E; ++e) s_part[wid * (D + 1) + lane * E + e] = acc[e];
-  if (lane == 0) s_part[wid * (D + 1) + D] = ls;
+  if (lane == 0) {
+    s_part[wid * (D + 1) + D] = ls;
+    s_red[wid] = M;
+  }
   __syncthreads();
   if (wid != 0) return;  // no barrier follows
-  float y[E];
-  const float lsum = (s_part[D] + s_part[(D + 1) + D]) + (s_part[2 * (D + 1) + D] + s_part[3 * (D + 1) + D]);
+  M = fmaxf(fmaxf(s_red[0], s_red[1]), fmaxf(s_red[2], s_red[3]));
+  float fw[4], y[E], lsum = 0.f;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    fw[w] = exp2f(s_red[w] - M);  // 0 for a wave without chunks
+    lsum = __builtin_fmaf(s_part[w * (D + 1) + D], fw[w], lsum);
+  }
   const float inv = 1.f / lsum;
 #pragma unroll
   for (int e = 0; e < E; ++e) {
-    const int j = lane * E + e;
-    y[e] = ((s_part[j] + s_part[(D + 1) + j]) + (s_part[2 * (D + 1) + j] + s_part[3 * (D + 1) + j])) * inv;
+    float o = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) o = __builtin_fmaf(s_part[w * (D + 1) + lane * E + e], fw[w], o);
+    y[e] = o * inv;
   }
   fwht_contig<E, 64, float>(y, lane);
   float* out = a.out + ((uint64_t)kv * a.nq + h) * D;
@@ -992,18 +1003,88 @@ hipError_t launch_nq(const AttnArgs& a, hipStream_t s) {
   return hipSuccess;
 }
 
+// Which calls the 16-bit matrix-core kernels (pitch_attn_codes.hip) take: the kind of caches, or -1.
+// They take key and value widths of 2, 3 and 4 bits, both codecs of one kind, and caches of which 64 token rows span
+// less than 2^31 bytes (a tile's rows are addressed with 32-bit offsets). Wider codes, whose tables would not fit the
+// LDS in 32 copies, keys and values of different per-vector methods, and enormous strides stay with this file's kernels.
+// So do the short calls of per-vector keys and values of equal width without the key-bias term, which attn_chunk
+// serves: the kernels' fixed cost (64 KB of table per workgroup) only pays from 32768 tokens over all KV heads at
+// d = 128 and 131072 at d = 64. Both sides there, us per call in a graph, b = 4: d = 128, 8 KV x 4 queries, 4096
+// tokens 12.2 here, 12.8 there; 6000 tokens 15.6 and 12.7; 2 KV x 4, 16384 tokens 13.6 and 14.6; 1 KV x 1, 65536
+// tokens 20.0 and 13.6; d = 64, 12 KV x 1, 8192 tokens 10.5 and 11.5; 16000 tokens 18.9 and 15.0. Up to 512 tokens
+// those calls go there too, since one workgroup then holds a KV head and there is no second launch (300 tokens, 8 KV x
+// 4: 11.9 and 10.0). Per-channel keys, the key-bias term and unequal widths take three or four launches here and are
+// faster there at every size (8 KV x 4, 300 tokens, per-channel: 14.2 and 9.7; 4096: 14.4 and 11.5).
+int codes_kind(const AttnArgs& a) {
+  if (a.kbits > 4 || a.vbits > 4) return -1;
+  if (a.token_stride > (1ull << 31) / (kTileTokens * PITCH_DIM)) return -1;
+  if (a.k_ranges) return a.vpolar ? kAttnKindChanPolar : kAttnKindChanTurbo;
+  if ((a.kpolar != 0) != (a.vpolar != 0)) return -1;
+  if (a.kb_cos) return a.kpolar ? kAttnKindPolarBias : kAttnKindTurboBias;
+  constexpr uint64_t kShort = PITCH_DIM == 128 ? 32768 : 131072;
+  if (a.kbits == a.vbits && a.tokens > 512 && a.tokens <= kShort / a.kv_heads) return -1;
+  return a.kpolar ? kAttnKindPolar : kAttnKindTurbo;
+}
+
+// Work split of the 16-bit matrix-core kernels: sets chunk (tokens per workgroup), chunks and the workspace regions,
+// returns the waves per workgroup (at least four: they also build the tables). A wave takes one 64-token tile at a
+// time. Up to 16 tiles (key-bias: 4) a KV head is one workgroup, which writes the output itself; longer calls take one
+// workgroup per compute unit, in multiples of eight chunks per KV head where there are so many (one for each XCD), of
+// at least two tiles (key-bias: one, since a workgroup's cos and sin rows are bound by what one compute unit reads:
+// 2 KV x 6, 2000 tokens 22.5 us with four, 18.1 with one), and at most 128 chunks, which attn_combine merges in two
+// rounds of loads.
+// The regions fit the workspace that a caller sizes with attention_workspace_floats, which holds, per padded query, 3 d
+// + tokens floats and 2 + d for every chunk of attn_chunk's (tests/test_attention_split.py).
+uint32_t codes_split(AttnArgs& a) {
+  const uint64_t tiles = (a.tokens + kTileTokens - 1) / kTileTokens;
+  const uint64_t cus = (uint64_t)device_cu_count();
+  const uint64_t fewest = a.kb_cos ? 1 : 2;
+  uint64_t chunks = 1;
+  if (tiles > (a.kb_cos ? 4 : kAttnCodesWaves)) {
+    chunks = cus / a.kv_heads;
+    if (chunks >= 8) chunks = chunks / 8 * 8;
+    const uint64_t most = (tiles + fewest - 1) / fewest;
+    chunks = chunks > most ? most : chunks > 128 ? 128 : chunks < 1 ? 1 : chunks;
+  }
+  const uint64_t per = (tiles + chunks - 1) / chunks;
+  a.chunk = (uint32_t)(per * kTileTokens);
+  a.chunks = (uint32_t)((tiles + per - 1) / per);
+  a.spread = a.chunks >= 8 && a.kv_heads > 1 && a.token_stride > 1;
+  a.ws_ml = 0;
+  a.ws_acc = (uint64_t)a.kv_heads * a.nqp * a.chunks * 2;
+  return (uint32_t)(per < 4 ? 4 : per < kAttnCodesWaves ? per : kAttnCodesWaves);
+}
+
+using CodesLaunch = hipError_t (*)(const AttnArgs&, uint32_t, hipStream_t);
+#define PITCH_CODES_CAT_(D, K) launch_attn_codes_d##D##_k##K
+#define PITCH_CODES_CAT(D, K) PITCH_CODES_CAT_(D, K)
+constexpr CodesLaunch kCodesLaunch[kAttnKinds] = {
+    PITCH_CODES_CAT(PITCH_DIM, 0), PITCH_CODES_CAT(PITCH_DIM, 1), PITCH_CODES_CAT(PITCH_DIM, 2),
+    PITCH_CODES_CAT(PITCH_DIM, 3), PITCH_CODES_CAT(PITCH_DIM, 4), PITCH_CODES_CAT(PITCH_DIM, 5)};
+
 }  // namespace
 
 #define PITCH_CAT2(a, b) a##b
 #define PITCH_CAT(a, b) PITCH_CAT2(a, b)
 
-hipError_t PITCH_CAT(launch_attention_d, PITCH_DIM)(const AttnArgs& a, hipStream_t s) {
+hipError_t PITCH_CAT(launch_attention_d, PITCH_DIM)(const AttnArgs& args, hipStream_t s) {
+  AttnArgs a = args;
   constexpr int D = PITCH_DIM;
   static_assert(D == 64 || D == 128, "attention dimensions");
   if (a.dim != (uint32_t)D || a.chunk < 64 || a.chunk > (uint32_t)kMaxChunk || a.chunks == 0) return hipErrorInvalidValue;
   if (a.k_ranges && (a.k_group == 0 || a.k_group % 64 != 0 || a.head_stride % a.k_group != 0 || a.token_stride != 1))
     return hipErrorInvalidValue;
   if (a.kb_cos && (a.k_ranges || !a.kb_bias || !a.kb_sin)) return hipErrorInvalidValue;
+  if (const int kind = codes_kind(a); kind >= 0) {
+    const uint32_t waves = codes_split(a);
+    const hipError_t ce = kCodesLaunch[kind](a, waves, s);
+    if (ce != hipSuccess) return ce;
+    if (a.chunks > 1) hipLaunchKernelGGL((attn_combine<D>), dim3(a.kv_heads * a.nq), dim3(kBlock), 0, s, a);
+    return hipGetLastError();
+  }
+  const WsLayout layout(a);
+  a.ws_ml = layout.ml;
+  a.ws_acc = layout.acc;
   // the scores kernels rotate the queries themselves (attn_rotates), with the key-bias term only in the
   // matrix-core form (attn_mfma)
   const bool rotate_inside = (a.nqp == 1 && attn_rotates<1>()) || (a.nqp == 2 && attn_rotates<2>()) ||

@@ -130,6 +130,8 @@ struct AttnArgs {
   uint32_t kv_heads;
   uint32_t kbits, vbits, kpolar, vpolar, kseed, vseed;
   uint32_t chunk, chunks;    // tokens per workgroup and chunks per KV head
+  uint32_t spread;           // 1: a chunk's KV heads on one XCD (pitch_attn_codes.hip)
+  uint64_t ws_ml, ws_acc;    // workspace regions (floats) of the chunks' (maximum, sum) and accumulators
   float qscale;              // softmax scale * log2(e) / sqrt(dim), folded into the rotated queries
   float oscale;              // 1 / sqrt(dim) of the value decode
   // Per-channel (KIVI) keys instead of per-vector ones (k_ranges non-null): codes [h][token] at

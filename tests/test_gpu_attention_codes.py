@@ -1,0 +1,133 @@
+"""The 16-bit matrix-core attention kernels (pitch_attn_codes.hip) at the sizes where their tiling can go wrong: one
+token, tiles of 64 tokens and their edges, one workgroup per KV head and the first sizes of several, chunks that end in
+a partial tile, and one to eight query heads (two row layouts), for each kind of caches and a width on every table path.
+
+Bar: 1e-5 relative L2 per query and 1e-5 on the log-sum-exp, as tests/test_gpu_attention.py derives it (float32
+accumulation; the kernels' own operands hold 22 bits and more). Values of very uneven scales keep the bar too: a
+token's weight is held relative to the largest scale in two parts of eleven bits, down to 2^-17 of it in full.
+"""
+import math
+
+import numpy as np
+import pytest
+
+from oracle import pitch_oracle as O
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-5
+
+
+def _packed(rng, kv, rows, d, bits):
+    codes = rng.integers(0, 2 ** bits, (kv, rows, d))
+    return codes, np.frombuffer(b"".join(O.pack_codes(c, bits) for c in codes), np.uint8).reshape(kv, rows, -1)
+
+
+def _compare(out, lse, ref_out, ref_lse, label):
+    for i in range(ref_out.shape[0]):
+        e = np.linalg.norm(out[i] - ref_out[i]) / np.linalg.norm(ref_out[i])
+        assert e < TOL, f"{label}: query {i} relative L2 {e}"
+    assert (np.abs(lse - ref_lse) / np.maximum(1.0, np.abs(ref_lse))).max() < TOL, label
+
+
+def _dev(q, *arrays):
+    import torch
+    return [torch.from_numpy(np.ascontiguousarray(a)).to(q.device) for a in arrays]
+
+
+# unequal widths reach the kernels at every length
+VECTOR = [("turboQuant", 4, 3, 128, 4, 2), ("turboQuant", 2, 4, 64, 1, 3), ("polarQuant", 3, 4, 128, 8, 1),
+          ("turboQuant", 3, 2, 64, 5, 2)]
+TOKENS = [1, 63, 64, 65, 1023, 1024, 1025, 1153, 8191, 20001]
+
+
+@pytest.mark.parametrize("tokens", TOKENS)
+@pytest.mark.parametrize("method,kb,vb,d,nq,kv", VECTOR)
+def test_vector_keys(q, method, kb, vb, d, nq, kv, tokens):
+    """Token-major caches; the values' scales span nine powers of two."""
+    import torch
+    import pitch_amd as P
+    label = f"{method} k{kb} v{vb} d={d} nq={nq} kv={kv} T={tokens}"
+    print(label, flush=True)
+    rng = np.random.default_rng(tokens + d + nq)
+    kc, kp = _packed(rng, kv, tokens, d, kb)
+    vc, vp = _packed(rng, kv, tokens, d, vb)
+    ks = np.exp(rng.uniform(1.5, 3.0, (kv, tokens))).astype(np.float32)
+    vs = np.exp2(rng.uniform(-4.0, 5.0, (kv, tokens))).astype(np.float32)
+    Q = rng.standard_normal((kv, nq, d)).astype(np.float32)
+    dq, dkc, dks, dvc, dvs = _dev(q, Q, kp.transpose(1, 0, 2), ks.T, vp.transpose(1, 0, 2), vs.T)
+    out, lse = torch.empty(kv, nq, d, device=q.device), torch.empty(kv, nq, device=q.device)
+    q.enqueueAttentionDecode(dq, dkc, dks, dvc, dvs, out, tokens, P.QuantConfig(method, d, kb, 101),
+                             P.QuantConfig(method, d, vb, 202), qPerKv=nq, kvHeads=kv, tokenStride=kv, headStride=1, lse=lse)
+    out, lse = out.cpu().numpy().astype(np.float64), lse.cpu().numpy().astype(np.float64)
+    for h in range(kv):
+        ro, rl = O.attention_decode(Q[h].astype(np.float64), kc[h], ks[h], vc[h], vs[h], method, kb, method, vb,
+                                    1 / math.sqrt(d), 101, 202)
+        _compare(out[h], lse[h], ro, rl, f"{label} head {h}")
+
+
+@pytest.mark.parametrize("tokens", TOKENS)
+@pytest.mark.parametrize("kb,vb,d,nq,kv,group", [(4, 3, 128, 4, 2, 64), (2, 2, 64, 8, 1, 128), (3, 4, 128, 6, 1, 64),
+                                                 (3, 3, 64, 2, 3, 64)])
+def test_channel_keys(q, kb, vb, d, nq, kv, group, tokens):
+    """Head-major per-channel keys with uneven channels, and a partial last group."""
+    import torch
+    import pitch_amd as P
+    label = f"channel k{kb} v{vb} d={d} nq={nq} kv={kv} G={group} T={tokens}"
+    print(label, flush=True)
+    rng = np.random.default_rng(tokens + d + nq + 7)
+    stride = -(-tokens // group) * group
+    K = (rng.standard_normal((kv, tokens, d)) * np.exp(rng.standard_normal((kv, 1, d))) + rng.standard_normal((kv, 1, d)))
+    groups = stride // group
+    kp = np.zeros((kv, stride, O.code_stride_bytes(d, kb)), np.uint8)
+    kr = np.zeros((kv, groups, 2, d), np.float16)
+    kcodes = []
+    for h in range(kv):
+        c, r = O.channel_encode(K[h].astype(np.float32), kb, group)
+        kcodes.append(c)
+        kp[h, :tokens] = np.frombuffer(O.pack_codes(c, kb), np.uint8).reshape(tokens, -1)
+        kr[h] = r
+    vc, vp = _packed(rng, kv, stride, d, vb)
+    vs = np.exp(rng.uniform(-1.0, 1.0, (kv, stride))).astype(np.float32)
+    Q = (0.5 * rng.standard_normal((kv, nq, d))).astype(np.float32)
+    dq, dkp, dkr, dvp, dvs = _dev(q, Q, kp, kr, vp, vs)
+    out, lse = torch.empty(kv, nq, d, device=q.device), torch.empty(kv, nq, device=q.device)
+    q.enqueueAttentionDecode(dq, dkp, dkr, dvp, dvs, out, tokens, P.ChannelQuantConfig(d, kb, group),
+                             P.QuantConfig("turboQuant", d, vb, 202), qPerKv=nq, kvHeads=kv, headStride=stride, lse=lse)
+    out, lse = out.cpu().numpy().astype(np.float64), lse.cpu().numpy().astype(np.float64)
+    for h in range(kv):
+        Kd = O.channel_decode(kcodes[h], kr[h], kb, group).astype(np.float64)
+        Vd = O.turbo_decode(vc[h, :tokens], vs[h, :tokens].astype(np.float64), vb, 202)
+        ro, rl = O.attend(Q[h].astype(np.float64), Kd, Vd, 1 / math.sqrt(d))
+        _compare(out[h], lse[h], ro, rl, f"{label} head {h}")
+
+
+@pytest.mark.parametrize("tokens", [1, 64, 65, 257, 4097])
+@pytest.mark.parametrize("method,kb,vb,d,nq,kv", [("turboQuant", 4, 4, 128, 6, 2), ("polarQuant", 3, 2, 64, 2, 3)])
+def test_key_bias(q, method, kb, vb, d, nq, kv, tokens):
+    import torch
+    import pitch_amd as P
+    label = f"bias {method} k{kb} v{vb} d={d} nq={nq} kv={kv} T={tokens}"
+    print(label, flush=True)
+    rng = np.random.default_rng(tokens + d + nq + 11)
+    first = 5
+    kc, kp = _packed(rng, kv, tokens, d, kb)
+    vc, vp = _packed(rng, kv, tokens, d, vb)
+    ks = np.exp(rng.uniform(1.5, 2.5, (kv, tokens))).astype(np.float32)
+    vs = np.exp(rng.uniform(-1.0, 1.0, (kv, tokens))).astype(np.float32)
+    ang = np.arange(first + tokens)[:, None] * (1e4 ** -(np.arange(d // 2) / (d // 2)))[None]
+    cos = np.concatenate([np.cos(ang)] * 2, 1).astype(np.float32)
+    sin = np.concatenate([np.sin(ang)] * 2, 1).astype(np.float32)
+    b = (3 * rng.standard_normal((kv, d))).astype(np.float32)
+    Q = (0.4 * rng.standard_normal((kv, nq, d))).astype(np.float32)
+    dq, dkc, dks, dvc, dvs, db, dcos, dsin = _dev(q, Q, kp.transpose(1, 0, 2), ks.T, vp.transpose(1, 0, 2), vs.T, b, cos, sin)
+    out, lse = torch.empty(kv, nq, d, device=q.device), torch.empty(kv, nq, device=q.device)
+    q.enqueueAttentionDecode(dq, dkc, dks, dvc, dvs, out, tokens, P.QuantConfig(method, d, kb, 101),
+                             P.QuantConfig(method, d, vb, 202), qPerKv=nq, kvHeads=kv, tokenStride=kv, headStride=1,
+                             lse=lse, keyBias=P.KeyBias(db, dcos, dsin, firstPosition=first, heads=kv))
+    out, lse = out.cpu().numpy().astype(np.float64), lse.cpu().numpy().astype(np.float64)
+    off = O.key_bias_offsets(b, cos, sin, first, tokens * kv, kv).reshape(tokens, kv, d).astype(np.float64)
+    for h in range(kv):
+        Kd = O.DECODERS[method](kc[h], ks[h].astype(np.float64), kb, 101) + off[:, h]
+        Vd = O.DECODERS[method](vc[h], vs[h].astype(np.float64), vb, 202)
+        ro, rl = O.attend(Q[h].astype(np.float64), Kd, Vd, 1 / math.sqrt(d))
+        _compare(out[h], lse[h], ro, rl, f"{label} head {h}")
