@@ -2064,7 +2064,7 @@ void vec_encode_hs_batch(VecBatchArgs pb) {
 }
 
 // ----------------------------------------------------------------------------------------------------
-// LDS-transposed encoder for float32 vectors at D = 256, 512 and 1024 (both methods). A vector is held by a
+// LDS-transposed encoder at D = 256, 512 and 1024 (both methods, every element type). A vector is held by a
 // team of T = D / 32 lanes, twice over:
 // - staging: team lane p loads the D / 32 chunks of CW = 1024 / D consecutive floats at coordinates
 //   CW p + 32 j (j = 0 .. T - 1; each load instruction reads 128 contiguous bytes of every vector), applies the
@@ -2123,32 +2123,58 @@ void fill_lt_flips(uint32_t seed, uint32_t* out) {
 #ifndef PITCH_LT_NTS
 #define PITCH_LT_NTS 1
 #endif
+// Loaded words of a lane's 32 coordinates: one each in float32 and where a 16-bit chunk is one element, else two
+// elements a word (widened to float32, exactly, when they are staged).
+template <int D, int IO>
+constexpr int lt_words() { return IO == 0 || Lt<D, false>::CW == 1 ? 32 : 16; }
+// (a macro: a template parameter would drop the 4-byte alignment of the vector types)
+#define PITCH_LT_LOAD(T, p) (PITCH_LT_NTL ? __builtin_nontemporal_load((const T*)(p)) : *(const T*)(p))
+
 // Loads of a wave's block of V vectors (vectors past the end re-read the last one).
-template <int D>
-__device__ __forceinline__ void lt_fetch(const float* in, uint64_t base, uint64_t count, int lane, uint32_t (&pf)[32]) {
+template <int D, int IO>
+__device__ __forceinline__ void lt_fetch(const void* in, uint64_t base, uint64_t count, int lane,
+                                         uint32_t (&pf)[lt_words<D, IO>()]) {
   using L = Lt<D, false>;
   const uint64_t v = base + lane / L::T;
-  const float* row = in + (v < count ? v : count - 1) * D + L::CW * (lane % L::T);
+  const char* row = (const char*)in + ((v < count ? v : count - 1) * D + L::CW * (lane % L::T)) * Io<IO>::kBytes;
+  constexpr int kBytes = L::CW * Io<IO>::kBytes, kStep = 32 * Io<IO>::kBytes;  // of a chunk; from chunk to chunk
 #pragma unroll
   for (int j = 0; j < L::NJ; ++j) {
-    if constexpr (L::CW == 4) {
-      const u32x4 c = PITCH_LT_NTL ? __builtin_nontemporal_load((const u32x4*)(row + 32 * j)) : *(const u32x4*)(row + 32 * j);
+    const char* p = row + kStep * j;
+    if constexpr (kBytes == 16) {
+      const u32x4 c = PITCH_LT_LOAD(u32x4, p);
       pf[4 * j] = c.x, pf[4 * j + 1] = c.y, pf[4 * j + 2] = c.z, pf[4 * j + 3] = c.w;
-    } else if constexpr (L::CW == 2) {
-      const u32x2 c = PITCH_LT_NTL ? __builtin_nontemporal_load((const u32x2*)(row + 32 * j)) : *(const u32x2*)(row + 32 * j);
+    } else if constexpr (kBytes == 8) {
+      const u32x2 c = PITCH_LT_LOAD(u32x2, p);
       pf[2 * j] = c.x, pf[2 * j + 1] = c.y;
+    } else if constexpr (kBytes == 4) {
+      pf[j] = PITCH_LT_LOAD(uint32_t, p);
     } else {
-      pf[j] = PITCH_LT_NTL ? __builtin_nontemporal_load((const uint32_t*)(row + 32 * j)) : *(const uint32_t*)(row + 32 * j);
+      pf[j] = PITCH_LT_LOAD(uint16_t, p);
     }
+  }
+}
+#undef PITCH_LT_LOAD
+// Element i of the lane's 32 (chunk i / CW, place i mod CW).
+template <int D, int IO>
+__device__ __forceinline__ float lt_element(const uint32_t (&pf)[lt_words<D, IO>()], int i) {
+  if constexpr (IO == 0) {
+    return __uint_as_float(pf[i]);
+  } else if constexpr (lt_words<D, IO>() == 32) {
+    return widen1<IO>((uint16_t)pf[i]);
+  } else {
+    float x[2];
+    widen2<IO>(pf[i / 2], x[0], x[1]);
+    return x[i & 1];
   }
 }
 
 // Staging of one block (see Lt): signs, float64, the stages on coordinate bits 5 and above, then two passes
 // through the wave's LDS rows, each for half of every vector's rows, after which lane q of a vector holds its
 // coordinates 32 q .. 32 q + 31 in x.
-template <int D, bool COLS>
-__device__ __forceinline__ void lt_stage(const uint32_t* neg, const uint32_t (&pf)[32], int lane, double* sx,
-                                         double (&x)[32]) {
+template <int D, bool COLS, int IO>
+__device__ __forceinline__ void lt_stage(const uint32_t* neg, const uint32_t (&pf)[lt_words<D, IO>()], int lane,
+                                         double* sx, double (&x)[32]) {
   using L = Lt<D, COLS>;
   constexpr int CW = L::CW, NJ = L::NJ, HR = L::HR;
   double y[NJ][CW];
@@ -2157,7 +2183,7 @@ __device__ __forceinline__ void lt_stage(const uint32_t* neg, const uint32_t (&p
 #pragma unroll
     for (int r = 0; r < CW; ++r) {
       const uint32_t m = neg[j * CW + r];
-      y[j][r] = (double)neg_lanes(__uint_as_float(pf[j * CW + r]), (uint64_t)m | ((uint64_t)m << 32));
+      y[j][r] = (double)neg_lanes(lt_element<D, IO>(pf, j * CW + r), (uint64_t)m | ((uint64_t)m << 32));
     }
 #pragma unroll
   for (int h = 1; h < NJ; h <<= 1)
@@ -2281,14 +2307,13 @@ __device__ __forceinline__ void lt_compute(const EncSeg& sg, const typename TqLu
 template <bool POLAR>
 constexpr int lt_waves() { return POLAR ? 3 : 2; }
 
-template <int D, int B, bool POLAR>
+template <int D, int B, bool POLAR, int IO>
 __device__ __forceinline__ void lt_run(const VecArgs& p, const EncSeg sg, uint64_t block, uint64_t nblocks) {
   using L = Lt<D, POLAR>;
   using Q = TqLut8<D, B>;
   __shared__ __attribute__((aligned(16))) double s_x[L::WAVES][L::ROWS];
   __shared__ __attribute__((aligned(16))) typename Q::Smem s_q;  // (unused by PolarQuant)
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const float* in = (const float*)sg.in;
   const uint64_t stride = nblocks * L::WAVES * L::V;
   uint64_t base = (block * L::WAVES + wave) * L::V;
   static_assert(!POLAR || sizeof(s_q) >= (size_t)OctTab<B>::N, "the octant table fits the bucket table's space");
@@ -2299,38 +2324,38 @@ __device__ __forceinline__ void lt_run(const VecArgs& p, const EncSeg sg, uint64
   const uint32_t* neg = p.lane_flips;  // fill_lt_flips; kernel arguments, read as scalars
   __syncthreads();
   if (base >= sg.count) return;
-  uint32_t pf[32];
-  lt_fetch<D>(in, base, sg.count, lane, pf);
+  uint32_t pf[lt_words<D, IO>()];
+  lt_fetch<D, IO>(sg.in, base, sg.count, lane, pf);
   double* sx = s_x[wave];
   double x[32];
   FairPriority fair(p.fair != 0, sg.count - base, stride);
-  lt_stage<D, POLAR>(neg, pf, lane, sx, x);
+  lt_stage<D, POLAR, IO>(neg, pf, lane, sx, x);
   while (base < sg.count) {
     fair.next();
-    lt_fetch<D>(in, base + stride, sg.count, lane, pf);
+    lt_fetch<D, IO>(sg.in, base + stride, sg.count, lane, pf);
     __builtin_amdgcn_sched_barrier(0);
     lt_compute<D, B, POLAR>(sg, s_q, base, lane, x);
     __builtin_amdgcn_sched_barrier(0);
     base += stride;
-    lt_stage<D, POLAR>(neg, pf, lane, sx, x);
+    lt_stage<D, POLAR, IO>(neg, pf, lane, sx, x);
   }
 }
 
-template <int D, int B, bool POLAR>
+template <int D, int B, bool POLAR, int IO>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(lt_waves<POLAR>())))
 void vec_encode_lt(VecArgs p) {
-  lt_run<D, B, POLAR>(p, call_segment(p), blockIdx.x, gridDim.x);
+  lt_run<D, B, POLAR, IO>(p, call_segment(p), blockIdx.x, gridDim.x);
 }
 
-template <int D, int B, bool POLAR>
+template <int D, int B, bool POLAR, int IO>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(lt_waves<POLAR>())))
 void vec_encode_lt_batch(VecBatchArgs pb) {
   const BatchSlot s = batch_slot(pb);
-  lt_run<D, B, POLAR>(pb.common, s.seg, s.block, s.blocks);
+  lt_run<D, B, POLAR, IO>(pb.common, s.seg, s.block, s.blocks);
 }
 
 #ifndef PITCH_LT_ENCODER
-#define PITCH_LT_ENCODER 1  // 1: float32 encode at D = 256 .. 1024 uses vec_encode_lt
+#define PITCH_LT_ENCODER 1  // 1: encode at D = 256 .. 1024 without key bias uses vec_encode_lt
 #endif
 
 #ifndef PITCH_HS_ENCODER
@@ -2357,9 +2382,21 @@ constexpr EncKind enc_kind() {
   if ((IO == 0 || (PITCH_HS_IO16 && !KBIAS && (POLAR || D == 128))) && (POLAR ? PITCH_HS_POLAR : PITCH_HS_ENCODER) &&
       (D == 64 || D == 128))
     return EncKind::kStaged;
-  if (IO == 0 && !KBIAS && PITCH_LT_ENCODER && D >= 256) return EncKind::kTransposed;
+  if (!KBIAS && PITCH_LT_ENCODER && D >= 256) return EncKind::kTransposed;
   if (!POLAR && use_lpv_encoder<D>()) return EncKind::kLanePerVector;
   return EncKind::kTeam;
+}
+// Whether a call of so many vectors runs the LDS-transposed encoder where enc_kind names it; the others run the team
+// encoder, with the same bytes. 16-bit TurboQuant takes it from 2^23 coordinates: below two of its resident rounds
+// (2 waves per SIMD against the team encoder's 4) its fixed cost loses. us per call, team and transposed, d = 256,
+// bfloat16: 64 vectors, b = 2: 4.4 and 5.2; 16744, b = 4: 7.7 and 9.3; 40000, b = 8: 13.8 and 13.5; 131072, b = 3: 41.0
+// and 31.8 (d = 512 and 1024 alike). PolarQuant gains at every size (the same four: 6.7 and 5.8, 12.9 and 11.0, 23.3
+// and 18.4, 68.8 and 35.1), float32 was measured faster before.
+template <int D, bool POLAR, int IO>
+constexpr bool lt_by_size() { return IO != 0 && !POLAR; }
+template <int D, bool POLAR, int IO>
+bool lt_pays(uint64_t vectors) {
+  return !lt_by_size<D, POLAR, IO>() || vectors >= (1u << 23) / D;
 }
 // Vectors a workgroup of that encoder (without key bias) takes per round.
 template <int D, bool POLAR, int IO>
@@ -2405,16 +2442,16 @@ hipError_t launch_one(bool encode, const VecArgs& args, hipStream_t s) {
     }
   }
   if constexpr (kEnc == EncKind::kTransposed) {
-    if (encode) {
+    if (encode && lt_pays<D, POLAR, IO>(a.count)) {
       using L = Lt<D, POLAR>;
       fill_lt_flips<D>(a.seed, a.lane_flips);
       const uint64_t need = (a.count + L::WAVES * L::V - 1) / (L::WAVES * L::V);
-      const void* k = (const void*)&vec_encode_lt<D, B, POLAR>;
+      const void* k = (const void*)&vec_encode_lt<D, B, POLAR, IO>;
       // persistent at every size: the oversubscribed grid of encode_grid measured 3-4 % slower on the d = 1024
       // sweep (2^20 vectors, 43 rounds)
       const uint64_t grid = persistent_grid(k, need);
       a.fair = need > grid ? 1u : 0u;
-      hipLaunchKernelGGL((vec_encode_lt<D, B, POLAR>), dim3((uint32_t)grid), dim3(kBlock), 0, s, a);
+      hipLaunchKernelGGL((vec_encode_lt<D, B, POLAR, IO>), dim3((uint32_t)grid), dim3(kBlock), 0, s, a);
       return hipGetLastError();
     }
   }
@@ -2432,9 +2469,11 @@ hipError_t launch_one(bool encode, const VecArgs& args, hipStream_t s) {
   fill_lane_flips<D>(a.seed, a.lane_flips);
   const uint64_t need = (a.count + G::VPB - 1) / G::VPB;
   if (encode) {
-    const void* k = (const void*)&vec_encode<D, B, POLAR, IO, KBIAS>;
-    const uint64_t grid = persistent_grid(k, need);
-    hipLaunchKernelGGL((vec_encode<D, B, POLAR, IO, KBIAS>), dim3((uint32_t)grid), dim3(kBlock), 0, s, a);
+    if constexpr (kEnc == EncKind::kTeam || (kEnc == EncKind::kTransposed && lt_by_size<D, POLAR, IO>())) {
+      const void* k = (const void*)&vec_encode<D, B, POLAR, IO, KBIAS>;
+      const uint64_t grid = persistent_grid(k, need);
+      hipLaunchKernelGGL((vec_encode<D, B, POLAR, IO, KBIAS>), dim3((uint32_t)grid), dim3(kBlock), 0, s, a);
+    }
   } else {
     // float32 calls of at least 2^19 vectors at d = 1024 (2 GB of output): the streaming decoder. At d = 128 one
     // workgroup per block of vec_decode (below) measured as fast as the streaming decoder at 2^25 vectors (config
@@ -2538,6 +2577,23 @@ template <int D, int B, bool POLAR>
 hipError_t launch_batch(VecBatchArgs a, hipStream_t s) {
   constexpr EncKind k = enc_kind<D, POLAR, PITCH_IO, false>();
   constexpr uint64_t vpb = enc_vectors_per_block<D, POLAR, PITCH_IO>();
+  uint64_t total = 0;
+  for (uint32_t j = 0; j < a.items; ++j) total += a.count[j];
+  if constexpr (k == EncKind::kTransposed) {
+    if (lt_pays<D, POLAR, PITCH_IO>(total)) {
+      const void* kp = (const void*)&vec_encode_lt_batch<D, B, POLAR, PITCH_IO>;
+      bool fair = false;
+      const dim3 grid(assign_blocks(a, vpb, [&](uint64_t t) {
+        const uint64_t g = persistent_grid(kp, t);
+        fair = t > g;
+        return g;
+      }));
+      a.common.fair = fair ? 1u : 0u;
+      fill_lt_flips<D>(a.common.seed, a.common.lane_flips);
+      hipLaunchKernelGGL((vec_encode_lt_batch<D, B, POLAR, PITCH_IO>), grid, dim3(kBlock), 0, s, a);
+      return hipGetLastError();
+    }
+  }
   if constexpr (k == EncKind::kStaged) {
     const void* kp = (const void*)&vec_encode_hs_batch<D, B, POLAR, PITCH_IO>;
     bool fair = false;  // a persistent grid of more than one round
@@ -2549,17 +2605,6 @@ hipError_t launch_batch(VecBatchArgs a, hipStream_t s) {
     a.common.fair = fair ? 1u : 0u;
     fill_hs_flips<D, hs_team<D>()>(a.common.seed, a.common.lane_flips);
     hipLaunchKernelGGL((vec_encode_hs_batch<D, B, POLAR, PITCH_IO>), grid, dim3(kBlock), 0, s, a);
-  } else if constexpr (k == EncKind::kTransposed) {
-    const void* kp = (const void*)&vec_encode_lt_batch<D, B, POLAR>;
-    bool fair = false;
-    const dim3 grid(assign_blocks(a, vpb, [&](uint64_t t) {
-      const uint64_t g = persistent_grid(kp, t);
-      fair = t > g;
-      return g;
-    }));
-    a.common.fair = fair ? 1u : 0u;
-    fill_lt_flips<D>(a.common.seed, a.common.lane_flips);
-    hipLaunchKernelGGL((vec_encode_lt_batch<D, B, POLAR>), grid, dim3(kBlock), 0, s, a);
   } else if constexpr (k == EncKind::kLanePerVector) {
     const void* kp = (const void*)&tq_encode_lpv_batch<D, B, PITCH_IO>;
     bool fair = false;
@@ -2570,9 +2615,9 @@ hipError_t launch_batch(VecBatchArgs a, hipStream_t s) {
     }));
     a.common.fair = fair ? 1u : 0u;
     hipLaunchKernelGGL((tq_encode_lpv_batch<D, B, PITCH_IO>), grid, dim3(64), 0, s, a);
-  } else {
+  } else if constexpr (k == EncKind::kTeam || lt_by_size<D, POLAR, PITCH_IO>()) {
     const void* kp = (const void*)&vec_encode_batch<D, B, POLAR, PITCH_IO>;
-    const dim3 grid(assign_blocks(a, vpb, [&](uint64_t t) { return persistent_grid(kp, t); }));
+    const dim3 grid(assign_blocks(a, Geom<D>::VPB, [&](uint64_t t) { return persistent_grid(kp, t); }));
     fill_lane_flips<D>(a.common.seed, a.common.lane_flips);
     hipLaunchKernelGGL((vec_encode_batch<D, B, POLAR, PITCH_IO>), grid, dim3(kBlock), 0, s, a);
   }
