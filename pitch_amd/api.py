@@ -504,6 +504,7 @@ def _buf(t, name: str):
     return t.data_ptr(), t.numel() * t.element_size()
 
 
+_IO_OF_DTYPE = None   # 16-bit torch dtypes' element type codes (built on first use: torch is imported lazily)
 _IO_NAMES = {"float32": _lib.IO_F32, "float16": _lib.IO_F16, "bfloat16": _lib.IO_BF16}
 
 
@@ -511,9 +512,12 @@ def _io_type(t, element_type=None) -> int:
     """Element type code (PITCH_IO_*) of an uncompressed buffer: element_type when given (a torch dtype or
     "float32" / "float16" / "bfloat16"), else the tensor's own dtype when it is float16 or bfloat16, else
     float32 (a raw byte buffer holds float32 values, as in the reference's untyped buffers)."""
-    torch = _torch()
     if element_type is None:
-        return {torch.float16: _lib.IO_F16, torch.bfloat16: _lib.IO_BF16}.get(t.dtype, _lib.IO_F32)
+        global _IO_OF_DTYPE
+        if _IO_OF_DTYPE is None:
+            torch = _torch()
+            _IO_OF_DTYPE = {torch.float16: _lib.IO_F16, torch.bfloat16: _lib.IO_BF16}
+        return _IO_OF_DTYPE.get(t.dtype, _lib.IO_F32)
     name = str(element_type).replace("torch.", "")
     if name not in _IO_NAMES:
         raise InvalidInput(f"element type {element_type} is not float32, float16 or bfloat16")
@@ -523,8 +527,8 @@ def _io_type(t, element_type=None) -> int:
 def _stream_handle(stream, device=None):
     """HIP stream handle: the given stream (an int handle or a torch stream), else torch's current stream of
     device (read with the raw query when torch has it: a fraction of a microsecond instead of about two)."""
-    torch = _torch()
     if stream is None:
+        torch = _torch()
         raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
         if raw is not None:
             idx = device.index if device is not None and device.index is not None else torch.cuda.current_device()
@@ -815,7 +819,6 @@ class PITCH:
         tokens rounded up to it).
         With keyBias (per-vector keys encoded with that key bias, pitch_enqueue_attention_decode_key_bias) the
         scores use decode(k) + R_t b: keyBias.heads must be kvHeads and token t sits at keyBias.firstPosition + t."""
-        torch = _torch()
         channel_keys = isinstance(keyConfig, ChannelQuantConfig)
         if channel_keys and valueConfig is None:
             raise InvalidInput("per-channel keys need a per-vector valueConfig")
@@ -831,6 +834,7 @@ class PITCH:
         if workspace is None and not noAlloc:
             nbytes = attention_workspace_bytes(valueConfig if channel_keys else keyConfig, valueConfig, tokens,
                                                qPerKv, kvHeads)
+            torch = _torch()
             workspace = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
         args = []
         for t, name in ((q, "query"), (keyCodes, "key codes"), (keyScales, "key scales"), (valueCodes, "value codes"),
@@ -936,6 +940,15 @@ class PITCH:
         _raise_for(rc)
 
 
+def _check_segment_field(v, name: str, least: int) -> None:
+    """A segment table's counts or offsets: one value, or one per segment."""
+    if type(v) is int and v >= least:    # one int in range needs no array (0.1 us against 1.3)
+        return
+    a = np.asarray(v)
+    if a.dtype.kind not in "iu" or (a < least).any():
+        raise InvalidInput(f"{name} {v!r} must be {'at least 1' if least else 'non-negative'}")
+
+
 class EncodeBatch:
     """A segment table for pitch_enqueue_encode_batch kept between calls: one segment per (input, codes, scales)
     buffer triple, e.g. one per layer's cache. Each enqueue sets the segments' counts and byte offsets in place
@@ -964,16 +977,12 @@ class EncodeBatch:
         return self._n
 
     def enqueue(self, count, inputOffsets=0, codesOffsets=0, scalesOffsets=0, stream=None) -> None:
-        for name, v in (("count", count), ("offset", inputOffsets), ("offset", codesOffsets),
-                        ("offset", scalesOffsets)):
-            a = np.asarray(v)
-            if a.dtype.kind not in "iu" or (a < (1 if name == "count" else 0)).any():
-                raise InvalidInput(f"{name} {v!r} must be {'at least 1' if name == 'count' else 'non-negative'}")
-        t = self._tab
-        t[:, 9] = count
-        t[:, 2] = inputOffsets
-        t[:, 5] = codesOffsets
-        t[:, 8] = scalesOffsets
+        values = ((9, count, "count", 1), (2, inputOffsets, "offset", 0), (5, codesOffsets, "offset", 0),
+                  (8, scalesOffsets, "offset", 0))
+        for column, v, name, least in values:
+            _check_segment_field(v, name, least)
+        for column, v, name, least in values:
+            self._tab[:, column] = v
         p = self._pitch
         _raise_for(p._lib.pitch_enqueue_encode_batch(ctypes.byref(self.config._c()), self._io, self._arr, self._n,
                                                      _stream_handle(stream, p.device)))
@@ -1007,16 +1016,12 @@ class DecodeBatch:
         return self._n
 
     def enqueue(self, count, codesOffsets=0, scalesOffsets=0, outputOffsets=0, stream=None) -> None:
-        for name, v in (("count", count), ("offset", codesOffsets), ("offset", scalesOffsets),
-                        ("offset", outputOffsets)):
-            a = np.asarray(v)
-            if a.dtype.kind not in "iu" or (a < (1 if name == "count" else 0)).any():
-                raise InvalidInput(f"{name} {v!r} must be {'at least 1' if name == 'count' else 'non-negative'}")
-        t = self._tab
-        t[:, 9] = count
-        t[:, 2] = codesOffsets
-        t[:, 5] = scalesOffsets
-        t[:, 8] = outputOffsets
+        values = ((9, count, "count", 1), (2, codesOffsets, "offset", 0), (5, scalesOffsets, "offset", 0),
+                  (8, outputOffsets, "offset", 0))
+        for column, v, name, least in values:
+            _check_segment_field(v, name, least)
+        for column, v, name, least in values:
+            self._tab[:, column] = v
         p = self._pitch
         _raise_for(p._lib.pitch_enqueue_decode_batch(ctypes.byref(self.config._c()), self._io, self._arr, self._n,
                                                      _stream_handle(stream, p.device)))
@@ -1026,6 +1031,8 @@ def _attention_desc(q_per_kv: int, kv_heads: int, tokens: int, token_stride: int
                     scale: float) -> _lib.PitchAttentionDescC:
     for name, v in (("qPerKv", q_per_kv), ("kvHeads", kv_heads), ("tokens", tokens), ("tokenStride", token_stride),
                     ("headStride", head_stride)):
+        if type(v) is int and v >= 0:
+            continue
         if not isinstance(v, (int, np.integer)) or v < 0:
             raise InvalidInput(f"{name} {v} must be a non-negative integer")
     return _lib.PitchAttentionDescC(int(q_per_kv), int(kv_heads), int(tokens), int(token_stride), int(head_stride),
@@ -1045,11 +1052,15 @@ def attention_workspace_bytes(keyConfig: QuantConfig, valueConfig: QuantConfig, 
 
 def _check_offsets(*offs) -> None:
     for o in offs:
+        if type(o) is int and o >= 0:   # nearly always: an eighth of the general test's time
+            continue
         if not isinstance(o, (int, np.integer)) or o < 0:
             raise InvalidInput(f"offset {o} must be a non-negative multiple of 4")
 
 
 def _count(c) -> int:
+    if type(c) is int and c >= 1:
+        return c
     if not isinstance(c, (int, np.integer)) or c < 1:
         raise InvalidInput("count must be at least 1")
     return int(c)
