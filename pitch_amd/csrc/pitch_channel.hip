@@ -226,7 +226,7 @@ constexpr int kSlab = PITCH_KIVI_DEC_SLAB;  // channels per wave of the decoder 
 #ifndef PITCH_KIVI_DEC_SLAB32_MAX
 #define PITCH_KIVI_DEC_SLAB32_MAX 32768
 #endif
-constexpr int kGroupMaxW = 64;   // largest group the wave encoder takes
+constexpr int kGroupMaxW = 128;  // largest group the wave encoder takes
 // Calls of the wave encoder and decoder longer than this many rounds (grid-stride iterations per workgroup) are
 // issued as several launches of this many rounds. At a 17 GB footprint (config 5 keys: 33.5M tokens, d = 128) a
 // single persistent launch reaches 4.4 TB/s encoding and 4.9 TB/s decoding; launches of 2 rounds reach 5.3 and
@@ -312,14 +312,18 @@ constexpr uint64_t kChanSliceRoundsDec = 1;
 // DP (direct packing; B = 2, 4 or 8 and a row width that is a multiple of SW): lane c's four codes of a token
 // are the byte-aligned bit-field [4 B c, 4 B c + 4 B) of the row's packed code stream, so the lane packs them
 // in registers and writes B / 2 bytes of packed row to LDS; the stores then copy packed rows.
-template <int B, int IO, int SW, bool DP>
+// GW: the most rows of a group, 32, 64 or 128 (with 32-channel slabs only, whose lanes then hold as many registers as
+// those of 64 x 64). Rows that a group does not have cost as much as those it has, so groups of at most 32 rows take 32:
+// 8 heads x 32768 tokens at d = 128, b = 4, bfloat16, groups of 32: 35.6 us with GW = 64, 24.0 with 32; groups of
+// 128: 41.7 us in chan_encode4, which reads the keys twice, 25.6 here (float32 55.0 and 29.3; 2048 tokens 12.5 and 4.4).
+template <int B, int IO, int SW, bool DP, int GW>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PITCH_KIVI_WAVES))) void chan_encode_w(ChanArgs p) {
   static_assert(!DP || B == 2 || B == 4 || B == 8, "direct packing needs byte-aligned lane fields");
   constexpr int QW = SW / 4;           // lanes per token row
   constexpr int RPI = 64 / QW;         // token rows per load instruction
-  constexpr int TPL = kGroupMaxW / RPI;  // tokens per lane
+  constexpr int TPL = GW / RPI;  // tokens per lane
   const float levels = (float)((1 << B) - 1);
-  __shared__ __attribute__((aligned(16))) uint8_t s_stage_all[kBlock / 64][kGroupMaxW * SW];
+  __shared__ __attribute__((aligned(16))) uint8_t s_stage_all[kBlock / 64][GW * SW];
   const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
   uint8_t* s_stage = s_stage_all[wid];
   const int r = lane / QW, c = lane % QW;
@@ -337,10 +341,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(PITCH_KI
     const uint64_t src = (uint64_t)first * dim + ch0 + (cact ? 4u * c : 0u);  // element index
 
     // loads: rows past the group's end re-read its last row (no effect on the range). In a group of all
-    // kGroupMaxW rows no row is clamped: each load is then a wave-uniform row base plus the lane's 32-bit byte
+    // GW rows no row is clamped: each load is then a wave-uniform row base plus the lane's 32-bit byte
     // offset, with no per-lane 64-bit address arithmetic.
     float4 x[TPL];
-    if (n == (uint32_t)kGroupMaxW) {
+    if (n == (uint32_t)GW) {
       constexpr uint32_t ES = IO == 0 ? 4u : 2u;  // bytes per key element
       const char* gbase = (const char*)p.in + ((uint64_t)first * dim + ch0) * ES;
       const uint32_t loff = (r * dim + (cact ? 4u * c : 0u)) * ES;
@@ -605,18 +609,19 @@ __global__ __launch_bounds__(kBlock) void chan_decode4(ChanArgs p) {
   }
 }
 
-// Group size a multiple of 64: one wave per (group, slab of SW channels), four independent waves per
-// workgroup. A lane loads the fp16 ranges of its CPL channels once, then for each 64-token chunk of the
+// Group size a multiple of 64, or 32: one wave per (group, slab of SW channels), four independent waves per
+// workgroup. A lane loads the fp16 ranges of its CPL channels once, then for each chunk of the
 // group issues all its code-word loads before decoding; lane (r, c) holds channels CPL c .. CPL c + CPL - 1 of
 // tokens r, r + 64 / TPL, ..., so one store instruction writes 64 CPL / SW whole slab rows. CPL = 8 (16-bit
 // output, B <= 4, a dimension of whole slabs only: every lane's eight channels exist) stores 16 bytes per lane
 // from one code word, as the float32 path's CPL = 4 does.
-template <int B, int SW, int IO, int CPL = 4>
+// CH: tokens per chunk, 64, or 32 for groups of 32 (wave_decodes_32).
+template <int B, int SW, int IO, int CPL = 4, int CH = 64>
 __global__ __launch_bounds__(kBlock) void chan_decode_w(ChanArgs p) {
   static_assert(CPL == 4 || (CPL == 8 && IO != 0 && B <= 4), "eight channels per lane: 16-bit output, one code word");
   constexpr int QW = SW / CPL;      // lanes per slab row
   constexpr int RPI = 64 / QW;      // rows per store instruction
-  constexpr int TPL = 64 / RPI;     // tokens per lane per 64-token chunk
+  constexpr int TPL = CH / RPI;     // tokens per lane per chunk
   constexpr uint32_t kMask = (1u << B) - 1u;
   const float levels = (float)((1 << B) - 1);
   const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -648,11 +653,11 @@ __global__ __launch_bounds__(kBlock) void chan_decode_w(ChanArgs p) {
     }
     const uint32_t pos = ch * B, wi = pos >> 5, sh = pos & 31u;
     const bool straddle = sh + (uint32_t)CPL * B > 32u;
-    for (uint32_t t0 = 0; t0 < n; t0 += 64) {
-      // float32 output, a full 64-token chunk of a full slab: every lane is active and no row is clamped, so each
+    for (uint32_t t0 = 0; t0 < n; t0 += CH) {
+      // float32 output, a full chunk of a full slab: every lane is active and no row is clamped, so each
       // load and store is a wave-uniform row base plus the lane's 32-bit byte offset (config-3 decode +5 %; with
       // 16-bit output the same path measured 5-7 % slower, so those keep the general path)
-      if (IO == 0 && n - t0 >= 64u && cw == (uint32_t)SW) {
+      if (IO == 0 && n - t0 >= (uint32_t)CH && cw == (uint32_t)SW) {
         constexpr uint32_t ES = 4u;  // bytes per output element
         const char* cb = (const char*)(p.codes_in + (uint64_t)(first + t0) * p.nwords);
         char* ob = (char*)p.out + ((uint64_t)(first + t0) * dim) * ES;
@@ -719,6 +724,16 @@ __global__ __launch_bounds__(kBlock) void chan_decode1(ChanArgs p) {
   }
 }
 
+// Whether a decode of 32-token groups runs the wave decoder in chunks of 32: every 16-bit call, and float32 calls of few
+// tokens. us per call, chan_decode4 and the wave decoder, b = 4: bfloat16, 8 heads x 32768 tokens, d = 64 15.0 and
+// 9.8, d = 80 19.1 and 17.4, d = 128 21.5 and 20.1; float32, 2048 tokens, d = 64 3.6 and 2.7, d = 128 3.4 and 2.7, but
+// 8 x 32768 tokens at d = 80 20.3 and 26.8, d = 128 26.3 and 30.7 (a lane's range set-up serves four rows only).
+// Other multiples of 32 keep chan_decode4 (groups of 96, d = 96, bfloat16, 4 x 20000 tokens: 18.2 and 22.7).
+template <int IO>
+bool wave_decodes_32(const ChanArgs& a) {
+  return a.group == 32u && (IO != 0 || a.count <= 16384u);
+}
+
 template <int B, int IO>
 hipError_t launch_b(bool encode, const ChanArgs& a, hipStream_t s) {
   const bool vec4 = (a.dim & 3u) == 0u;
@@ -729,13 +744,13 @@ hipError_t launch_b(bool encode, const ChanArgs& a, hipStream_t s) {
     // 64-channel slabs, whose loads read whole 256-byte rows (+4 % at 131072 items). With 16-bit keys a
     // 64-channel row is only 128 bytes and the wider slab measured 6-7 % faster at 4096 items as well.
     const uint64_t items64 = groups * ((a.dim + 63) / 64);
-    const int sw = PITCH_KIVI_SLAB ? PITCH_KIVI_SLAB : (IO == 0 && items64 <= 32768 ? 32 : 64);
+    const int sw = a.group > 64u ? 32 : PITCH_KIVI_SLAB ? PITCH_KIVI_SLAB : (IO == 0 && items64 <= 32768 ? 32 : 64);
     const bool dp = PITCH_KIVI_DP && (B == 2 || B == 4 || B == 8) && a.dim % (uint32_t)sw == 0u;  // full slabs
-    auto go = [&](auto sw_c, auto dp_c) {
-      constexpr int SW = decltype(sw_c)::value;
+    auto go = [&](auto sw_c, auto dp_c, auto gw_c) {
+      constexpr int SW = decltype(sw_c)::value, GW = decltype(gw_c)::value;
       constexpr bool DP = decltype(dp_c)::value;
       const uint64_t items = groups * ((a.dim + SW - 1) / SW);
-      const void* k = (const void*)&chan_encode_w<B, IO, SW, DP>;
+      const void* k = (const void*)&chan_encode_w<B, IO, SW, DP, GW>;
       // float32 keys: balanced rounds (config 3 is 1.33 rounds at full occupancy); the 16-bit encoders are
       // bound by their arithmetic and keep every resident wave
       const uint64_t grid = persistent_grid(k, (items + 3) / 4, kBlock, PITCH_KIVI_BALANCE && IO == 0);
@@ -747,7 +762,7 @@ hipError_t launch_b(bool encode, const ChanArgs& a, hipStream_t s) {
         // hold (config-5 keys, 341 rounds: 5.52 TB/s against 5.41 for launches of two rounds, three repeats each,
         // before the cap), held at cap workgroups per CU (0: the kernel's full residency)
         const uint64_t g = need < 0x7FFFFFFFull ? need : 0x7FFFFFFFull;
-        hipLaunchKernelGGL((chan_encode_w<B, IO, SW, DP>), dim3((uint32_t)g), dim3(kBlock),
+        hipLaunchKernelGGL((chan_encode_w<B, IO, SW, DP, GW>), dim3((uint32_t)g), dim3(kBlock),
                            lds_cap_bytes(k, cap), s, a);
         return;
       }
@@ -763,22 +778,33 @@ hipError_t launch_b(bool encode, const ChanArgs& a, hipStream_t s) {
           b.codes_out = a.codes_out + t0 * a.nwords;
           b.ranges_out = a.ranges_out + g0 * 2 * a.dim;
           const uint64_t gb = ((uint64_t)b.count + a.group - 1) / a.group, nb = (gb * slabs + 3) / 4;
-          hipLaunchKernelGGL((chan_encode_w<B, IO, SW, DP>), dim3((uint32_t)(nb < grid ? nb : grid)), dim3(kBlock), 0,
+          hipLaunchKernelGGL((chan_encode_w<B, IO, SW, DP, GW>), dim3((uint32_t)(nb < grid ? nb : grid)), dim3(kBlock), 0,
                              s, b);
         }
         return;
       }
-      hipLaunchKernelGGL((chan_encode_w<B, IO, SW, DP>), dim3((uint32_t)grid), dim3(kBlock), 0, s, a);
+      hipLaunchKernelGGL((chan_encode_w<B, IO, SW, DP, GW>), dim3((uint32_t)grid), dim3(kBlock), 0, s, a);
     };
     using I32 = std::integral_constant<int, 32>;
     using I64 = std::integral_constant<int, 64>;
     constexpr bool kDP = B == 2 || B == 4 || B == 8;
-    if (sw == 32) {
-      if (dp) go(I32{}, std::integral_constant<bool, kDP>{});
-      else go(I32{}, std::false_type{});
+    using G32 = std::integral_constant<int, 32>;
+    using G64 = std::integral_constant<int, 64>;
+    using G128 = std::integral_constant<int, 128>;
+    auto rows = [&](auto sw_c, auto dp_c) {
+      if (a.group <= 32u) go(sw_c, dp_c, G32{});
+      else go(sw_c, dp_c, G64{});
+    };
+    using Packed = std::integral_constant<bool, kDP>;
+    if (a.group > 64u) {
+      if (dp) go(I32{}, Packed{}, G128{});
+      else go(I32{}, std::false_type{}, G128{});
+    } else if (sw == 32) {
+      if (dp) rows(I32{}, Packed{});
+      else rows(I32{}, std::false_type{});
     } else {
-      if (dp) go(I64{}, std::integral_constant<bool, kDP>{});
-      else go(I64{}, std::false_type{});
+      if (dp) rows(I64{}, Packed{});
+      else rows(I64{}, std::false_type{});
     }
   } else if (encode) {
     const uint64_t groups = ((uint64_t)a.count + a.group - 1) / a.group;
@@ -786,22 +812,22 @@ hipError_t launch_b(bool encode, const ChanArgs& a, hipStream_t s) {
     const uint64_t grid = persistent_grid(k, groups);
     if (vec4) hipLaunchKernelGGL((chan_encode4<B, IO>), dim3((uint32_t)grid), dim3(kBlock), 0, s, a);
     else hipLaunchKernelGGL((chan_encode1<B, IO>), dim3((uint32_t)grid), dim3(kBlock), 0, s, a);
-  } else if (vec4 && a.group % 64u == 0u) {
+  } else if (vec4 && (a.group % 64u == 0u || wave_decodes_32<IO>(a))) {
     // float32 output: 32-channel slabs for calls with few (group, 64-channel) items, which then fill the
     // resident waves (config-3 decode +3-4 % back-to-back, within 0.5 % in kernel time); 16-bit output keeps
     // 64-channel slabs (a 32-channel slab's rows are 64 bytes: 22 % slower)
     const uint64_t groups = ((uint64_t)a.count + a.group - 1) / a.group;
     const uint64_t items64 = groups * ((a.dim + kSlab - 1) / kSlab);
-    auto go = [&](auto sw_c, auto cpl_c) {
-      constexpr int SW = decltype(sw_c)::value, CPL = decltype(cpl_c)::value;
+    auto go = [&](auto sw_c, auto cpl_c, auto ch_c) {
+      constexpr int SW = decltype(sw_c)::value, CPL = decltype(cpl_c)::value, CH = decltype(ch_c)::value;
       const uint64_t items = groups * ((a.dim + SW - 1) / SW);
-      const uint64_t grid = persistent_grid((const void*)&chan_decode_w<B, SW, IO, CPL>, (items + 3) / 4);
+      const uint64_t grid = persistent_grid((const void*)&chan_decode_w<B, SW, IO, CPL, CH>, (items + 3) / 4);
       if (IO == 0 && PITCH_KIVI_DEC_ONE_LAUNCH && (items + 3) / 4 >= PITCH_KIVI_DEC_MIN_ROUNDS * grid) {
         // one launch of one item per wave at a capped residency (above); the kernel's grid-stride loop covers
         // any items past 2^31 - 1 workgroups
         const uint64_t need = (items + 3) / 4, g = need < 0x7FFFFFFFull ? need : 0x7FFFFFFFull;
-        const void* k = (const void*)&chan_decode_w<B, SW, IO, CPL>;
-        hipLaunchKernelGGL((chan_decode_w<B, SW, IO, CPL>), dim3((uint32_t)g), dim3(kBlock),
+        const void* k = (const void*)&chan_decode_w<B, SW, IO, CPL, CH>;
+        hipLaunchKernelGGL((chan_decode_w<B, SW, IO, CPL, CH>), dim3((uint32_t)g), dim3(kBlock),
                            lds_cap_bytes(k, PITCH_KIVI_DEC_WG_PER_CU), s, a);
         return;
       }
@@ -817,21 +843,27 @@ hipError_t launch_b(bool encode, const ChanArgs& a, hipStream_t s) {
           b.ranges_in = a.ranges_in + g0 * 2 * a.dim;
           b.out = (char*)a.out + t0 * a.dim * ES;
           const uint64_t gb = ((uint64_t)b.count + a.group - 1) / a.group, nb = (gb * slabs + 3) / 4;
-          hipLaunchKernelGGL((chan_decode_w<B, SW, IO, CPL>), dim3((uint32_t)(nb < grid ? nb : grid)), dim3(kBlock), 0, s, b);
+          hipLaunchKernelGGL((chan_decode_w<B, SW, IO, CPL, CH>), dim3((uint32_t)(nb < grid ? nb : grid)), dim3(kBlock), 0, s, b);
         }
         return;
       }
-      hipLaunchKernelGGL((chan_decode_w<B, SW, IO, CPL>), dim3((uint32_t)grid), dim3(kBlock), 0, s, a);
+      hipLaunchKernelGGL((chan_decode_w<B, SW, IO, CPL, CH>), dim3((uint32_t)grid), dim3(kBlock), 0, s, a);
     };
     // 16-bit output at B <= 4 with whole slabs, long calls: eight channels per lane (16-byte stores from one code
     // word); same output bits as four
     constexpr int kCpl16 = IO != 0 && B <= 4 && PITCH_KIVI_DEC_CPL8 ? 8 : 4;
     using Cpl4 = std::integral_constant<int, 4>;
-    if (PITCH_KIVI_DEC_SLAB32 && IO == 0 && items64 <= PITCH_KIVI_DEC_SLAB32_MAX)
-      go(std::integral_constant<int, 32>{}, Cpl4{});
+    using C32 = std::integral_constant<int, 32>;
+    using C64 = std::integral_constant<int, 64>;
+    using Slab = std::integral_constant<int, kSlab>;
+    const bool narrow = PITCH_KIVI_DEC_SLAB32 && IO == 0 && items64 <= PITCH_KIVI_DEC_SLAB32_MAX;
+    if (a.group % 64u != 0u) {
+      if (narrow) go(std::integral_constant<int, 32>{}, Cpl4{}, C32{});
+      else go(Slab{}, Cpl4{}, C32{});
+    } else if (narrow) go(std::integral_constant<int, 32>{}, Cpl4{}, C64{});
     else if (kCpl16 == 8 && a.dim % kSlab == 0u && items64 >= PITCH_KIVI_DEC_CPL8_MIN_ITEMS)
-      go(std::integral_constant<int, kSlab>{}, std::integral_constant<int, kCpl16>{});
-    else go(std::integral_constant<int, kSlab>{}, Cpl4{});
+      go(Slab{}, std::integral_constant<int, kCpl16>{}, C64{});
+    else go(Slab{}, Cpl4{}, C64{});
   } else if (vec4) {
     const uint32_t P = kBlock / (a.dim >> 2);
     const uint64_t need = ((uint64_t)a.count + P * kDecR - 1) / (P * kDecR);

@@ -1,0 +1,37 @@
+"""Per-channel encode and decode at the group sizes where the wave kernels change: 32, 64 and 128 rows for the encoder,
+32- and 64-token chunks for the decoder, and the sizes around them, with whole, partial and single-token last groups.
+Codes, ranges and decoded values are the oracle's bits (zero extremes of both signs included)."""
+import numpy as np
+import pytest
+
+from oracle import pitch_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("io", ["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize("group", [1, 17, 31, 32, 33, 63, 65, 96, 100, 127, 128, 129, 160])
+@pytest.mark.parametrize("dim,bits", [(64, 4), (80, 3), (96, 2), (128, 8), (36, 5)])
+def test_bits(q, dim, bits, group, io):
+    import torch
+    print(f"d={dim} b={bits} G={group} {io}", flush=True)
+    rng = np.random.default_rng(dim * 1000 + group)
+    tokens = 3 * group + (group + 1) // 2
+    x = rng.standard_normal((tokens, dim)).astype(np.float32) * np.exp(rng.standard_normal(dim)).astype(np.float32)
+    x[:, 3] = np.abs(x[:, 3])
+    x[rng.random(tokens) < 0.3, 3] = -0.0
+    x[rng.random(tokens) < 0.3, 3] = 0.0        # a minimum of either zero
+    t = torch.from_numpy(x).to(getattr(torch, io))
+    wide = t.float().numpy()
+    codes, ranges = O.channel_encode(wide, bits, group)
+    cfg = q.channelConfig(dim, bits, group)
+    dev = t.to(q.device)
+    c = torch.zeros(tokens * cfg.codeStride, dtype=torch.uint8, device=q.device)
+    r = torch.zeros(ranges.size, dtype=torch.int16, device=q.device)
+    q.enqueuePerChannelEncode(dev, c, r, tokens, cfg)
+    assert c.cpu().numpy().tobytes() == O.pack_codes(codes, bits)
+    assert np.array_equal(r.cpu().numpy().view(np.uint16), ranges.reshape(-1).view(np.uint16))
+    out = torch.zeros((tokens, dim), dtype=t.dtype, device=q.device)
+    q.enqueuePerChannelDecode(c, r, out, tokens, cfg)
+    want = O.to_io_bits(O.channel_decode(codes, ranges, bits, group), io)
+    assert np.array_equal(out.cpu().view(torch.int32 if io == "float32" else torch.int16).numpy().view(want.dtype), want)
