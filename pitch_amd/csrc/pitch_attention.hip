@@ -19,6 +19,8 @@
 //   attn_combine  merges the chunks, divides by the softmax sum, inverse rotation, output and log-sum-exp
 // With equal key and value bit widths attn_chunk runs the scores and values phases in one kernel and keeps the
 // weights p in LDS (attn_scores and attn_values remain for unequal widths and for per-channel keys).
+// Most calls with widths of 2 - 4 bits run attn_codes instead of all but attn_combine (pitch_attn_codes.hip; the rule
+// is codes_kind below).
 // Query heads of one KV head (grouped-query attention) share every table read; their count is padded to
 // 1, 2, 4 or 8 (padded queries are zero and never written out). With 4 or 8 the scores' and the values' products
 // run on the matrix cores (v_mfma_f32_4x4x1f32, below).

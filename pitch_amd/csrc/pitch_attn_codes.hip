@@ -13,21 +13,23 @@
 //   * the other operand (rotated queries, softmax weights) is split too, its parts on rows that the few query heads
 //     of a KV head leave empty: row 4 part + head for up to four heads (three parts of the query, two of the
 //     weights), row 8 part + head for up to eight (two parts). The parts' products are summed in float32.
-// The error against float64 is 0.5 to 1.0 of attn_chunk's over the widths, methods and sizes above (two float16 parts
-// hold a table value to 2^-23, three a query to 2^-33, and the score is rounded once where its maximum is subtracted).
+// Two float16 parts hold a table value to 2^-23, three a query to 2^-33. Error against float64 (relative L2, mean of
+// ten seeds), attn_chunk's -> this kernel's: 8 KV x 4 queries, 16000 tokens 6.9e-7 -> 4.9e-7; key-bias term, 2 KV x 6,
+// 2000 tokens 1.1e-6 -> 7.0e-7; per-channel keys 0.6 - 1.8e-6 -> 2.7 - 8.5e-7.
 // Per-channel keys need no table: a code is exact in bfloat16, so a group's query products q_j step_j are split into
 // three bfloat16 parts (24 bits) and the codes are converted in registers (v_mfma_f32_16x16x32_bf16).
 //
 // Work split: a wave takes tiles of 64 tokens by itself (scores, online softmax, weighted values), so no barrier
 // separates the phases and the waves of a SIMD hide each other's loads; a workgroup's waves merge through LDS at the
-// end and attn_combine merges the workgroups. Accumulators are added up per tile in float32 on the VALU: the matrix
-// cores truncate what they align to a running sum, which a long chain would feel.
+// end and attn_combine merges the workgroups. Weighted values are added up per tile, scores of table keys per two steps,
+// in float32 on the VALU: the matrix cores truncate what they align to a running sum, which a long chain would feel
+// (one chain per score: mean 6.3e-7 and at most 1.35e-6 of ten seeds, pairs of steps 4.9e-7 and 6.2e-7; same time).
 //
 // Bound: long calls by their reads (Llama-3-8B layer, 8 KV x 4 queries, b = 4, token-major: 131072 tokens 64 -> 43 us,
-// 3.3 TB/s; without its table reads and products the kernel takes as long, without its loads 24 us less 14), the rest
-// by fixed latency: launch, tables, one tile and the second launch are 10 - 12 us. Same layer: 16000 tokens 23.2 ->
-// 13.7, 32768 tokens 23.0 -> 17.6; per-channel keys of four bits and values of three, 131072 tokens 74.8 -> 41;
-// key-bias term, 2 KV x 6, 2000 tokens 22.0 -> 18.8, 4 KV x 4, 48606 tokens 210 -> 35.
+// 3.3 TB/s; with every tile read from the same few, so out of L2, 8 us less, without the loads 16 less), the rest by
+// fixed latency: launch, tables, one tile and the second launch are 10 - 12 us. Same layer: 16000 tokens 23.2 -> 13.7,
+// 32768 tokens 23.0 -> 17.6; per-channel keys of four bits and values of three, 131072 tokens 72.8 -> 42; key-bias
+// term, 2 KV x 6, 2000 tokens 21.8 -> 18.5, 4 KV x 4, 48606 tokens 210 -> 35.
 #include "pitch_attn_shared.h"
 
 #ifndef PITCH_DIM
@@ -522,7 +524,8 @@ __global__ __launch_bounds__(64 * max_waves(Q8)) void attn_codes(AttnArgs a) {
     const bool in = (uint32_t)lane < nt - tile * kTile;  // this lane's token is one of the chunk's
 
     // ---- scores: c[m] of lane (n, g) = rows 4 g .. 4 g + 3 (parts and heads) of token 16 m + n
-    v4f cs[4];
+    // (table keys: pairs of steps start from zero and are added on the VALU, see above)
+    v4f cs[4], co[4];
 #pragma unroll
     for (int m = 0; m < 4; ++m) cs[m] = v4f{0.f, 0.f, 0.f, 0.f};
     if constexpr (GC * KB % 32 != 0) {
@@ -618,8 +621,15 @@ __global__ __launch_bounds__(64 * max_waves(Q8)) void attn_codes(AttnArgs a) {
         if (k + 1 < 2 * KS) look(k + 1);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int m = 0; m < 2; ++m) cs[2 * (k & 1) + m] = mfma_f16(qa[(k >> 1) & 1], t[k & 1][m], cs[2 * (k & 1) + m]);
+        for (int m = 0; m < 2; ++m) {
+          v4f& sum = co[2 * (k & 1) + m];
+          sum = mfma_f16(qa[(k >> 1) & 1], t[k & 1][m], (k >> 1) & 1 ? sum : v4f{0.f, 0.f, 0.f, 0.f});
+        }
         __builtin_amdgcn_sched_barrier(0);
+        if ((k >> 1) & 1) {
+#pragma unroll
+          for (int m = 0; m < 2; ++m) cs[2 * (k & 1) + m] += co[2 * (k & 1) + m];
+        }
       }
     }
     float s[NH];
