@@ -169,6 +169,12 @@ constexpr uint32_t top_bits(int k) {
   return x;
 }
 
+// b where the mask's bits are set, a elsewhere. (A choice between two elements of a private array by a lane's condition
+// is compiled into an indexed load, which puts the array into scratch memory.)
+__device__ __forceinline__ float pick(uint32_t mask, float a, float b) {
+  return __uint_as_float((__float_as_uint(a) & ~mask) | (__float_as_uint(b) & mask));
+}
+
 // (x & mask) | rest in one instruction.
 __device__ __forceinline__ uint32_t and_or(uint32_t x, uint32_t mask, uint32_t rest) {
   uint32_t r;
@@ -496,6 +502,7 @@ __global__ __launch_bounds__(64 * max_waves(Q8)) void attn_codes(AttnArgs a) {
 #pragma unroll
   for (int i = 0; i < NA; ++i) acc[i] = v4f{0.f, 0.f, 0.f, 0.f};
   const uint32_t even = n < 8 ? ~0u : 0u;  // this lane weighs (row n) a pair's first coordinate
+  const uint32_t odd = g & 1 ? ~0u : 0u;   // eight heads: this lane accumulates heads 4 - 7
   int ev = -100;  // exponent of the values' scales that the accumulators are stored relative to
 
   // Key-bias term: a tile's cos rows, then its sin rows, in steps of 32 coordinates, loaded two steps ahead of their
@@ -729,7 +736,7 @@ __global__ __launch_bounds__(64 * max_waves(Q8)) void attn_codes(AttnArgs a) {
     float fr[4];
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      if constexpr (Q8) fr[v] = (g & 1) ? f[4 + v] : f[v];
+      if constexpr (Q8) fr[v] = pick(odd, f[v], f[4 + v]);
       else fr[v] = uniform(f[v]);
     }
 
