@@ -942,7 +942,7 @@ class PITCH:
 
 def _check_segment_field(v, name: str, least: int) -> None:
     """A segment table's counts or offsets: one value, or one per segment."""
-    if type(v) is int and v >= least:    # one int in range needs no array (0.1 us against 1.3)
+    if type(v) is int and least <= v < 1 << 64:    # one int that a field holds needs no array (0.1 us against 1.3)
         return
     a = np.asarray(v)
     if a.dtype.kind not in "iu" or (a < least).any():

@@ -277,3 +277,18 @@ def test_product_never_imports_the_oracle():
     for f in list(pkg.rglob("*.py")):
         text = f.read_text()
         assert "oracle" not in text, f"{f} mentions the oracle"
+
+
+# ----------------------------------------------------------------------------- batch tables
+@pytest.mark.parametrize("cls,fields", [(P.EncodeBatch, ("inputOffsets", "codesOffsets", "scalesOffsets")),
+                                        (P.DecodeBatch, ("codesOffsets", "scalesOffsets", "outputOffsets"))])
+@pytest.mark.parametrize("bad", [-1, 1 << 64, 1 << 200, True, 1.0, [4, -4], [4, 1 << 64]])
+def test_batch_table_refuses_before_it_writes(cls, fields, bad):
+    """Counts and offsets that a segment's 64-bit fields cannot hold are refused as InvalidInput, and a refused call
+    leaves the table as it was."""
+    batch = object.__new__(cls)
+    batch._tab = np.full((2, 10), 7, np.uint64)
+    for name in ("count",) + fields:
+        with pytest.raises(P.InvalidInput):
+            batch.enqueue(**{"count": 1, **{f: 8 for f in fields}, name: bad})
+        assert (batch._tab == 7).all()
