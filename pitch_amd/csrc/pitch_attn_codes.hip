@@ -875,21 +875,21 @@ __global__ __launch_bounds__(64 * max_waves(Q8)) void attn_codes(AttnArgs a) {
   }
 }
 
-// Lets a kernel take more than 64 KB of LDS (a property of the kernel: nothing is launched).
-hipError_t allow_lds(const void* kernel, uint32_t bytes) {
-  return bytes <= 65536u ? hipSuccess
-                         : hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-}
-
 template <int KB, int VB, bool Q8>
 hipError_t launch_one(const AttnArgs& a, uint32_t waves, hipStream_t s) {
   using S = Shape<PITCH_DIM, KB, VB, Q8>;
-  static_assert(S::bytes(max_waves(Q8)) <= 160u * 1024u, "LDS of one workgroup");
+  constexpr uint32_t kMostBytes = S::bytes(max_waves(Q8));
+  static_assert(kMostBytes <= 160u * 1024u, "LDS of one workgroup");
   waves = waves < max_waves(Q8) ? waves : max_waves(Q8);
   const uint32_t bytes = S::bytes(waves);
-  const void* k = (const void*)attn_codes<PITCH_DIM, KB, VB, Q8>;
-  const hipError_t e = allow_lds(k, bytes);
-  if (e != hipSuccess) return e;
+  // More than 64 KB of LDS have to be allowed for the kernel. That is a property of the kernel, not of the launch, so
+  // every call sets what the largest launch takes: a value of its own could be lowered by a shorter call of another
+  // thread between this call's setting and its launch.
+  if (bytes > 65536u) {
+    const hipError_t e = hipFuncSetAttribute((const void*)attn_codes<PITCH_DIM, KB, VB, Q8>,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMostBytes);
+    if (e != hipSuccess) return e;
+  }
   hipLaunchKernelGGL((attn_codes<PITCH_DIM, KB, VB, Q8>), dim3(a.spread ? (a.chunks + 7) / 8 * 8 * a.kv_heads : a.chunks * a.kv_heads), dim3(64 * waves), bytes, s, a);
   return hipSuccess;
 }

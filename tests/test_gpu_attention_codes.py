@@ -131,3 +131,51 @@ def test_key_bias(q, method, kb, vb, d, nq, kv, tokens):
         Vd = O.DECODERS[method](vc[h], vs[h].astype(np.float64), vb, 202)
         ro, rl = O.attend(Q[h].astype(np.float64), Kd, Vd, 1 / math.sqrt(d))
         _compare(out[h], lse[h], ro, rl, f"{label} head {h}")
+
+
+def test_threads_of_different_lengths(q):
+    """Calls of one kernel variant from several threads, each on a stream of its own, with lengths that take four waves
+    a workgroup and sixteen (different amounts of LDS): none is refused and each writes what it writes alone."""
+    import threading
+
+    import torch
+    import pitch_amd as P
+    d, nq, kv = 128, 4, 2
+    rng = np.random.default_rng(5)
+    kcfg, vcfg = P.QuantConfig("turboQuant", d, 4, 101), P.QuantConfig("turboQuant", d, 3, 202)
+
+    def call(tokens):
+        _, kp = _packed(rng, kv, tokens, d, 4)
+        _, vp = _packed(rng, kv, tokens, d, 3)
+        ks, vs = (np.exp(rng.uniform(0.0, 1.0, (kv, tokens))).astype(np.float32) for _ in range(2))
+        args = _dev(q, rng.standard_normal((kv, nq, d)).astype(np.float32), kp, ks, vp, vs)
+        ws = torch.empty(P.attention_workspace_bytes(kcfg, vcfg, tokens, nq, kv), dtype=torch.uint8, device=q.device)
+
+        def run(out, stream=None):
+            q.enqueueAttentionDecode(*args, out, tokens, kcfg, vcfg, qPerKv=nq, kvHeads=kv, workspace=ws, stream=stream)
+        alone = torch.empty(kv, nq, d, device=q.device)
+        run(alone)
+        return run, alone
+
+    calls = [call(t) for t in (200, 1024, 100, 900)]
+    torch.cuda.synchronize()
+    failed = []
+
+    def work(run, alone):
+        try:
+            stream = torch.cuda.Stream()
+            outs = [torch.full_like(alone, float("nan")) for _ in range(8)]
+            torch.cuda.synchronize()
+            for i in range(400):
+                run(outs[i % 8], stream)
+            stream.synchronize()
+            assert all(torch.equal(o, alone) for o in outs)
+        except Exception as e:  # noqa: BLE001 (reported by the main thread)
+            failed.append(repr(e))
+
+    threads = [threading.Thread(target=work, args=c) for c in calls]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed, failed
