@@ -149,3 +149,29 @@ def test_batch_with_an_invalid_segment_launches_nothing(q):
         q.enqueueEncodeBatch([], cfg)
     with pytest.raises(P.InvalidInput):
         q.enqueueEncodeBatch([segs[0], (x.half(), codes, scales, n)], cfg)   # mixed element types
+
+
+def test_batch_of_many_allocations(q):
+    """Twelve segments whose caches are allocations of their own (4 MB and more each): all are written, and a host
+    address in the last segment is refused before anything is."""
+    import torch
+    import pitch_amd as P
+    dev, n, segments = q.device, 3, 12
+    cfg = P.QuantConfig("turboQuant", 128, 4)
+    x = [torch.randn(n, 128, device=dev) for _ in range(segments)]
+    codes = [torch.zeros(4 << 20, dtype=torch.uint8, device=dev) for _ in range(segments)]
+    scales = [torch.zeros(1 << 20, device=dev) for _ in range(segments)]
+    tab = P.EncodeBatch(q, cfg, x, codes, scales)
+    host = np.zeros(4 << 20, np.uint8)
+    good = tab._arr[segments - 1].codes
+    tab._arr[segments - 1].codes = host.ctypes.data
+    with pytest.raises(P.InvalidInput, match="codes"):
+        tab.enqueue(n)
+    torch.cuda.synchronize()
+    assert not any(t.any() for t in codes + scales)
+    tab._arr[segments - 1].codes = good
+    tab.enqueue(n)
+    for i in range(segments):
+        rc, rs = torch.zeros(n * cfg.codeStride, dtype=torch.uint8, device=dev), torch.zeros(n, device=dev)
+        q.enqueueEncode(x[i], rc, rs, n, cfg)
+        assert torch.equal(codes[i][:n * cfg.codeStride], rc) and torch.equal(scales[i][:n], rs)
