@@ -359,6 +359,14 @@ int pitch_enqueue_unpack_codes(uint32_t dim, uint32_t bits, const void* packed, 
  * the number that differ (0 expected) to *mismatches. For tests and bring-up on new hardware. */
 int pitch_selftest_reciprocal(uint64_t* mismatches);
 
+/* Self-test of the work split of attention over codes of 2-4 bits, without a device; no counterpart in the
+ * reference. For a call of kv_heads heads x tokens with one query head per KV head on a device of compute_units, writes
+ * the tokens per workgroup, the workgroups per KV head (each leaves 2 + dim floats of partial results in the workspace
+ * when there are several), the waves per workgroup and the floats of the workspace that
+ * pitch_attention_workspace_size asks for (workspace_chunk 0; otherwise of one sized with chunks of that many tokens). */
+int pitch_selftest_attention_split(uint32_t dim, uint64_t tokens, uint32_t kv_heads, uint32_t key_bias,
+                                   uint32_t compute_units, uint32_t workspace_chunk, uint64_t split[4]);
+
 #ifdef __cplusplus
 }
 #endif

@@ -11,6 +11,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
+#include <algorithm>
 #include <mutex>
 #include <vector>
 #include <string>
@@ -575,6 +576,30 @@ uint64_t attention_workspace_floats(uint32_t dim, uint32_t nqp, uint32_t kv_head
   return (uint64_t)kv_heads * nqp * (3 * dim + tokens + chunks * (2 + dim));
 }
 
+// A wave takes one 64-token tile at a time. Up to 16 tiles (key-bias: 4) a KV head is one workgroup, which writes the
+// output itself; longer calls take one workgroup per compute unit, in multiples of eight chunks per KV head where there
+// are so many (one for each XCD), of at least two tiles (key-bias: one, since a workgroup's cos and sin rows are bound
+// by what one compute unit reads: 2 KV x 6, 2000 tokens 22.5 us with four, 18.1 with one), and at most 128 chunks,
+// which attn_combine merges in two rounds of loads (one KV head, 30000 tokens, per-channel keys: 16.5 us with 235, 13.6 with 118).
+// The partials of all chunks fit the caller's workspace by construction: it holds 3 d + tokens floats per padded query
+// and 2 + d for every chunk of ws_chunk tokens (attention_workspace_floats).
+CodesSplit attention_codes_split(uint32_t dim, uint64_t tokens, uint32_t kv_heads, bool key_bias, uint32_t cus,
+                                 uint32_t ws_chunk) {
+  const uint64_t tiles = (tokens + kTileTokens - 1) / kTileTokens;
+  const uint64_t fewest = key_bias ? 1 : 2;
+  uint64_t chunks = 1;
+  if (tiles > (key_bias ? 4u : kAttnCodesWaves)) {
+    chunks = cus / kv_heads;
+    if (chunks >= 8) chunks = chunks / 8 * 8;
+    chunks = std::min<uint64_t>({chunks, (tiles + fewest - 1) / fewest, kAttnMostChunks});
+    chunks = std::max<uint64_t>(chunks, (tiles >> 24) + 1);  // a chunk's tokens are counted in 32 bits
+    chunks = std::min<uint64_t>(chunks, attention_workspace_floats(dim, 1, 1, tokens, ws_chunk) / (2 + dim));
+  }
+  const uint64_t per = (tiles + chunks - 1) / chunks;
+  return {(uint32_t)(per * kTileTokens), (uint32_t)((tiles + per - 1) / per),
+          (uint32_t)(per < 4 ? 4 : per < kAttnCodesWaves ? per : kAttnCodesWaves)};  // four at least build the tables
+}
+
 uint64_t slice_rounds(uint64_t dflt) { return PITCH_SLICE_ROUNDS >= 0 ? (uint64_t)PITCH_SLICE_ROUNDS : dflt; }
 
 uint64_t stream_decode_min_vectors() { return (uint64_t)PITCH_STREAM_MIN_VECTORS; }
@@ -1135,6 +1160,21 @@ int pitch_selftest_reciprocal(uint64_t* mismatches) {
   uint64_t total = 0;
   for (uint32_t c : h) total += c;
   *mismatches = total;
+  return ok();
+}
+
+int pitch_selftest_attention_split(uint32_t dim, uint64_t tokens, uint32_t kv_heads, uint32_t key_bias,
+                                   uint32_t compute_units, uint32_t workspace_chunk, uint64_t split[4]) {
+  if (!split) return fail(PITCH_ERR_INVALID_INPUT, "split is null");
+  if (dim == 0 || tokens == 0 || kv_heads == 0)
+    return fail(PITCH_ERR_INVALID_INPUT, "dimension, tokens and KV heads must be at least 1");
+  const uint32_t chunk = workspace_chunk ? workspace_chunk : pitch::attention_chunk_tokens(tokens, kv_heads);
+  const pitch::CodesSplit x =
+      pitch::attention_codes_split(dim, tokens, kv_heads, key_bias != 0, compute_units, chunk);
+  split[0] = x.chunk;
+  split[1] = x.chunks;
+  split[2] = x.waves;
+  split[3] = pitch::attention_workspace_floats(dim, 1, kv_heads, tokens, chunk);
   return ok();
 }
 

@@ -1028,33 +1028,16 @@ int codes_kind(const AttnArgs& a) {
   return a.kpolar ? kAttnKindPolar : kAttnKindTurbo;
 }
 
-// Work split of the 16-bit matrix-core kernels: sets chunk (tokens per workgroup), chunks and the workspace regions,
-// returns the waves per workgroup (at least four: they also build the tables). A wave takes one 64-token tile at a
-// time. Up to 16 tiles (key-bias: 4) a KV head is one workgroup, which writes the output itself; longer calls take one
-// workgroup per compute unit, in multiples of eight chunks per KV head where there are so many (one for each XCD), of
-// at least two tiles (key-bias: one, since a workgroup's cos and sin rows are bound by what one compute unit reads:
-// 2 KV x 6, 2000 tokens 22.5 us with four, 18.1 with one), and at most 128 chunks, which attn_combine merges in two
-// rounds of loads.
-// The regions fit the workspace that a caller sizes with attention_workspace_floats, which holds, per padded query, 3 d
-// + tokens floats and 2 + d for every chunk of attn_chunk's (tests/test_attention_split.py).
+// Sets a call's work split (attention_codes_split) and workspace regions, returns the waves per workgroup.
 uint32_t codes_split(AttnArgs& a) {
-  const uint64_t tiles = (a.tokens + kTileTokens - 1) / kTileTokens;
-  const uint64_t cus = (uint64_t)device_cu_count();
-  const uint64_t fewest = a.kb_cos ? 1 : 2;
-  uint64_t chunks = 1;
-  if (tiles > (a.kb_cos ? 4 : kAttnCodesWaves)) {
-    chunks = cus / a.kv_heads;
-    if (chunks >= 8) chunks = chunks / 8 * 8;
-    const uint64_t most = (tiles + fewest - 1) / fewest;
-    chunks = chunks > most ? most : chunks > 128 ? 128 : chunks < 1 ? 1 : chunks;
-  }
-  const uint64_t per = (tiles + chunks - 1) / chunks;
-  a.chunk = (uint32_t)(per * kTileTokens);
-  a.chunks = (uint32_t)((tiles + per - 1) / per);
+  const CodesSplit x = attention_codes_split(a.dim, a.tokens, a.kv_heads, a.kb_cos != nullptr,
+                                             (uint32_t)device_cu_count(), a.chunk);
+  a.chunk = x.chunk;
+  a.chunks = x.chunks;
   a.spread = a.chunks >= 8 && a.kv_heads > 1 && a.token_stride > 1;
   a.ws_ml = 0;
   a.ws_acc = (uint64_t)a.kv_heads * a.nqp * a.chunks * 2;
-  return (uint32_t)(per < 4 ? 4 : per < kAttnCodesWaves ? per : kAttnCodesWaves);
+  return x.waves;
 }
 
 using CodesLaunch = hipError_t (*)(const AttnArgs&, uint32_t, hipStream_t);

@@ -16,8 +16,6 @@ constexpr float kLn2 = 0x1.62e430p-1f;   // ln(2)
 #define kAttnKindChanTurbo 4  // per-channel keys, TurboQuant values
 #define kAttnKindChanPolar 5  // per-channel keys, PolarQuant values
 constexpr int kAttnKinds = 6;
-constexpr uint32_t kTileTokens = 64;     // tokens a wave takes at a time
-constexpr uint32_t kAttnCodesWaves = 16;  // most waves per workgroup
 
 #define PITCH_DECLARE_ATTN_CODES(K)                                                          \
   hipError_t launch_attn_codes_d64_k##K(const AttnArgs& a, uint32_t waves, hipStream_t s);   \

@@ -150,6 +150,17 @@ struct AttnArgs {
 // Chunk length (tokens per workgroup) the attention kernels use for a call, and the workspace it needs.
 uint32_t attention_chunk_tokens(uint64_t tokens, uint32_t kv_heads);
 uint64_t attention_workspace_floats(uint32_t dim, uint32_t nqp, uint32_t kv_heads, uint64_t tokens, uint32_t chunk);
+
+// Work split of the 16-bit matrix-core kernels (pitch_attn_codes.hip): tokens per workgroup, workgroups (chunks) per KV
+// head, waves per workgroup. ws_chunk is the chunk length that the call's workspace was sized with.
+constexpr uint32_t kTileTokens = 64;      // tokens a wave takes at a time
+constexpr uint32_t kAttnCodesWaves = 16;  // most waves per workgroup
+constexpr uint32_t kAttnMostChunks = 128;
+struct CodesSplit {
+  uint32_t chunk, chunks, waves;
+};
+CodesSplit attention_codes_split(uint32_t dim, uint64_t tokens, uint32_t kv_heads, bool key_bias, uint32_t cus,
+                                 uint32_t ws_chunk);
 hipError_t launch_attention_d64(const AttnArgs& a, hipStream_t s);
 hipError_t launch_attention_d128(const AttnArgs& a, hipStream_t s);
 

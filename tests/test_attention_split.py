@@ -1,40 +1,49 @@
-"""The work split of the 16-bit matrix-core attention kernels (codes_split in pitch_attention.hip) against the
-workspace that pitch_attention_workspace_size promises its callers: restated here, since a launch needs a GPU."""
+"""The work split of the 16-bit matrix-core attention kernels, as the library computes it for a launch
+(pitch_selftest_attention_split): every chunk's partial results fit the workspace that callers are told to bring, on
+devices of any size and for a workspace sized with any chunk length, and the split covers the tokens."""
 import ctypes
 
 import pytest
 
 from pitch_amd import _lib
 
-
-def codes_chunks(tokens: int, kv: int, bias: bool, cus: int) -> int:
-    tiles = -(-tokens // 64)
-    chunks = 1
-    if tiles > (4 if bias else 16):
-        chunks = cus // kv
-        if chunks >= 8:
-            chunks = chunks // 8 * 8
-        most = tiles if bias else -(-tiles // 2)
-        chunks = min(chunks, most) if chunks > most else min(max(chunks, 1), 128)
-    per = -(-tiles // chunks)
-    return -(-tiles // per)
+EDGES = sorted({2 ** k + e for k in range(5, 22) for e in (-1, 0, 1, 63, 64, 65)} | set(range(1, 1400, 7))
+               | {2 ** 32 - 1, 2 ** 32, 2 ** 36})
 
 
-@pytest.mark.parametrize("bias", [False, True])
-@pytest.mark.parametrize("dim", [64, 128])
-def test_partials_fit_the_workspace(dim, bias):
-    if not _lib.LIB_PATH.exists():
-        pytest.skip("HIP library not built")
+@pytest.fixture(scope="module")
+def split(built_library):
     lib = _lib.load()
-    cfg = _lib.PitchConfigC(0, dim, 4, 1)
-    out = ctypes.c_uint64()
-    edges = {2 ** k + e for k in range(5, 22) for e in (-1, 0, 1, 63, 64, 65)} | set(range(1, 1400, 7))
-    for cus in (1, 64, 256, 304):
-        for kv in (1, 2, 3, 8, 12, 200):
-            for tokens in sorted(edges):
-                desc = _lib.PitchAttentionDescC(1, kv, tokens, 1, tokens, 1.0, 0)
-                assert lib.pitch_attention_workspace_size(ctypes.byref(cfg), ctypes.byref(cfg), ctypes.byref(desc),
-                                                          ctypes.byref(out)) == 0
-                chunks = codes_chunks(tokens, kv, bias, cus)
+    out = (ctypes.c_uint64 * 4)()
+
+    def call(dim, tokens, kv, bias, cus, ws_chunk=0):
+        assert lib.pitch_selftest_attention_split(dim, tokens, kv, bias, cus, ws_chunk, out) == 0
+        return tuple(out)
+    return call
+
+
+@pytest.mark.parametrize("ws_chunk", [0, 64, 128, 1024])
+@pytest.mark.parametrize("bias", [0, 1])
+@pytest.mark.parametrize("dim", [64, 128])
+def test_partials_fit_the_workspace(split, dim, bias, ws_chunk):
+    for cus in (1, 64, 256, 304, 1024):
+        for kv in (1, 2, 3, 8, 12, 48, 129, 200, 300, 65535):
+            for tokens in EDGES:
+                chunk, chunks, waves, floats = split(dim, tokens, kv, bias, cus, ws_chunk)
+                label = (cus, kv, tokens, chunk, chunks)
+                assert chunk % 64 == 0 and chunk < 2 ** 31 and (chunks - 1) * chunk < tokens <= chunks * chunk, label
+                assert chunks <= 128 and 4 <= waves <= 16, label
                 if chunks > 1:    # a single chunk writes the output itself
-                    assert 4 * kv * chunks * (2 + dim) <= out.value, (cus, kv, tokens, chunks)
+                    assert kv * chunks * (2 + dim) <= floats, label
+
+
+def test_workspace_is_what_the_size_query_says(split):
+    lib = _lib.load()
+    cfg = _lib.PitchConfigC(0, 128, 4, 1)
+    size = ctypes.c_uint64()
+    for kv in (1, 3, 64):
+        for tokens in (1, 1000, 70000):
+            desc = _lib.PitchAttentionDescC(1, kv, tokens, 1, tokens, 1.0, 0)
+            assert lib.pitch_attention_workspace_size(ctypes.byref(cfg), ctypes.byref(cfg), ctypes.byref(desc),
+                                                      ctypes.byref(size)) == 0
+            assert size.value == 4 * split(128, tokens, kv, 0, 256)[3]
