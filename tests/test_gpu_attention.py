@@ -105,6 +105,30 @@ def test_attention_against_oracle(q, k_method, v_method, kb, vb, d, nq, kv, T):
         _check(out[h], lse[h], ro, rl, OUT_REL_L2, LSE_TOL, f"{label} head {h}")
 
 
+@pytest.mark.parametrize("T", [128, 129, 8192, 8193, 16385, 40000])
+@pytest.mark.parametrize("d,bits,nq", [(64, 5, 2), (128, 6, 4)])
+def test_attention_chunk_counts(q, d, bits, nq, T):
+    """One KV head in chunks of 128 tokens, merged in one round of loads (64 chunks, T = 8192) and in several; the
+    largest score lies in the first chunk for half of the queries and in the last for the others."""
+    import torch
+    import pitch_amd as P
+    print(f"chunks d={d} b={bits} nq={nq} T={T}", flush=True)
+    rng = np.random.default_rng(T + d)
+    kc, kp, ks = _random_cache(rng, 1, T, d, bits, 1.5, 3.0)
+    vc, vp, vs = _random_cache(rng, 1, T, d, bits, -1.0, 1.0)
+    K = O.turbo_decode(kc[0], ks[0].astype(np.float64), bits, 101)
+    Q = np.stack([K[0 if i % 2 else T - 1] * 0.15 for i in range(nq)])[None].astype(np.float32)
+    cfg, dev = P.QuantConfig("turboQuant", d, bits, 101), q.device
+    out, lse = torch.empty(1, nq, d, device=dev), torch.empty(1, nq, device=dev)
+    q.enqueueAttentionDecode(torch.from_numpy(Q).to(dev), torch.from_numpy(kp.copy()).to(dev),
+                             torch.from_numpy(ks).to(dev), torch.from_numpy(vp.copy()).to(dev),
+                             torch.from_numpy(vs).to(dev), out, T, cfg, qPerKv=nq, lse=lse)
+    torch.cuda.synchronize()
+    ro, rl = O.attention_decode(Q[0].astype(np.float64), kc[0], ks[0], vc[0], vs[0], "turboQuant", bits, "turboQuant",
+                                bits, 1 / math.sqrt(d), 101, 101)
+    _check(out.cpu().numpy()[0], lse.cpu().numpy()[0], ro, rl, OUT_REL_L2, LSE_TOL, f"chunks T={T}")
+
+
 @pytest.mark.parametrize("d", [64, 128])
 def test_attention_peaky_scores(q, d):
     """Sharp softmax: scale 12 / sqrt(d) puts the largest scores near 40."""
