@@ -111,6 +111,18 @@ __device__ __forceinline__ void wave_max4(const float (&x)[4], float (&m)[4]) {
   m[2] = lane_value(r, 16);
   m[3] = lane_value(r, 48);
 }
+// The same of every head's value.
+template <int NH>
+__device__ __forceinline__ void wave_max_heads(const float (&x)[NH], float (&m)[NH]) {
+#pragma unroll
+  for (int h = 0; h < NH; h += 4) {
+    const float x4[4] = {x[h], x[h + 1], x[h + 2], x[h + 3]};
+    float m4[4];
+    wave_max4(x4, m4);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) m[h + k] = m4[k];
+  }
+}
 __device__ __forceinline__ float wave_sum(float x) {
   x += xchg<1>(x);
   x += xchg<2>(x);
@@ -258,7 +270,7 @@ struct Shape {
   static constexpr int KOPS = kChanKeys && Q8 ? 2 : 1;  // operands of a group's query products (the third part of eight)
   static constexpr int kW = 2 * NH * kWRow, kAcc = NH * D, kGq = kChanKeys ? KOPS * KS * 256 : 0;
   static constexpr int kWave = kW > kAcc ? (kW > kGq ? kW : kGq) : (kAcc > kGq ? kAcc : kGq);
-  static constexpr int kStat = 2 * NH + 16;      // per wave: maxima, sums, value exponent
+  static constexpr int kStat = 2 * NH + 16;      // per wave: maxima, sums (and the tables' constants before)
   static constexpr int kHead = 2 * NH;          // per head: the query operand's and the bias operand's scale
   __host__ __device__ static constexpr uint32_t bytes(uint32_t waves) {
     return 4u * (uint32_t)(kTabK + kTabV + kQ + kBiasQ + kHead) + 4u * waves * (uint32_t)(kWave + kStat);
@@ -503,7 +515,6 @@ __global__ __launch_bounds__(64 * max_waves(Q8)) void attn_codes(AttnArgs a) {
   for (int i = 0; i < NA; ++i) acc[i] = v4f{0.f, 0.f, 0.f, 0.f};
   const uint32_t even = n < 8 ? ~0u : 0u;  // this lane weighs (row n) a pair's first coordinate
   const uint32_t odd = g & 1 ? ~0u : 0u;   // eight heads: this lane accumulates heads 4 - 7
-  int ev = -100;  // exponent of the values' scales that the accumulators are stored relative to
 
   // Key-bias term: a tile's cos rows, then its sin rows, in steps of 32 coordinates, loaded two steps ahead of their
   // products (the first two ahead of the tile's scores).
@@ -698,47 +709,39 @@ __global__ __launch_bounds__(64 * max_waves(Q8)) void attn_codes(AttnArgs a) {
     const uint32_t next = more ? tile + (uint32_t)waves : tile;
     load_keys(next, more ? min(nt - 1u - next * kTile, (uint32_t)kTile - 1u) : 0u);
 
-    // ---- online softmax; weights p n_t relative to the running maximum and to 2^ev, in two float16 parts
-    float fe = 1.f;
+    // ---- online softmax; the tile's weights w = p n_t relative to the largest of them per head, in two float16 parts
     const float n_t = in ? nv : 0.f;
-    if (__builtin_amdgcn_ballot_w64(exponent_of(n_t) > ev)) {
-      const int grown = max(exponent_of(wave_max(__builtin_fabsf(n_t))), ev);
-      fe = pow2i(max(ev - grown, -126));
-      ev = grown;
-    }
-    const float nvs = n_t * pow2i(14 - ev);
-    float sv[NH], mx[NH], f[NH];
+    float sv[NH], mx[NH], al[NH], w[NH], fx[NH];
 #pragma unroll
     for (int h = 0; h < NH; ++h) sv[h] = in ? __builtin_fmaf(s[h], sf[h], sb[h]) : -__builtin_inff();
-#pragma unroll
-    for (int h = 0; h < NH; h += 4) {
-      const float x[4] = {sv[h], sv[h + 1], sv[h + 2], sv[h + 3]};
-      float m[4];
-      wave_max4(x, m);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) mx[h + k] = m[k];
-    }
+    wave_max_heads(sv, mx);
 #pragma unroll
     for (int h = 0; h < NH; ++h) {
       const float m = uniform(fmax_hw(M[h], mx[h]));
-      const float al = __builtin_amdgcn_exp2f(M[h] - m);
+      al[h] = __builtin_amdgcn_exp2f(M[h] - m);
       M[h] = m;
       const float p = in ? __builtin_amdgcn_exp2f(__builtin_fmaf(s[h], sf[h], sb[h] - m)) : 0.f;
-      l[h] = __builtin_fmaf(l[h], al, p);
-      f[h] = al * fe;
-      const float w = p * nvs;
-      const _Float16 hi = (_Float16)w;
-      const _Float16 lo = (_Float16)((w - (float)hi) * kLoScale);
+      l[h] = __builtin_fmaf(l[h], al[h], p);
+      w[h] = p * n_t;
+      sv[h] = __builtin_fabsf(w[h]);
+    }
+    float fa[4], ft[4];  // factors of the accumulators and of the tile's sums
+#pragma unroll
+    for (int v = 0; v < 4; ++v) fa[v] = Q8 ? pick(odd, al[v], al[NH - 4 + v]) : al[v];
+    wave_max_heads(sv, mx);
+#pragma unroll
+    for (int h = 0; h < NH; ++h) {
+      const int e = max(exponent_of(mx[h]), -100);
+      fx[h] = pow2i(e - 14 - 12);  // 2^14 of the weights, 2^12 of the table
+      const float y = w[h] * pow2i(14 - e);
+      const _Float16 hi = (_Float16)y;
+      const _Float16 lo = (_Float16)((y - (float)hi) * kLoScale);
       s_w[h * kWRow + lane] = twice(hi);
       s_w[(NH + h) * kWRow + lane] = twice(lo);
     }
     wave_lds_fence();
-    float fr[4];
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      if constexpr (Q8) fr[v] = pick(odd, f[v], f[4 + v]);
-      else fr[v] = uniform(f[v]);
-    }
+    for (int v = 0; v < 4; ++v) ft[v] = Q8 ? pick(odd, fx[v], fx[NH - 4 + v]) : fx[v];
 
     // ---- weighted values. A step takes two tokens of each lane group and a code pair, whose two values lie side by
     // side on the contraction axis as the table read returns them; the weights are zero at the other value's place:
@@ -796,10 +799,10 @@ __global__ __launch_bounds__(64 * max_waves(Q8)) void attn_codes(AttnArgs a) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         if constexpr (Q8) {
-          acc[2 * p][v] = __builtin_fmaf(acc[2 * p][v], fr[v], x[p][v]);
-          acc[2 * p + 1][v] = __builtin_fmaf(acc[2 * p + 1][v], fr[v], y[p][v]);
+          acc[2 * p][v] = __builtin_fmaf(acc[2 * p][v], fa[v], x[p][v] * ft[v]);
+          acc[2 * p + 1][v] = __builtin_fmaf(acc[2 * p + 1][v], fa[v], y[p][v] * ft[v]);
         } else {
-          acc[p][v] = __builtin_fmaf(acc[p][v], fr[v], x[p][v]);
+          acc[p][v] = __builtin_fmaf(acc[p][v], fa[v], x[p][v] * ft[v]);
         }
       }
     wave_lds_fence();
@@ -815,7 +818,6 @@ __global__ __launch_bounds__(64 * max_waves(Q8)) void attn_codes(AttnArgs a) {
       st[h] = M[h];
       st[NH + h] = l[h];
     }
-    st[2 * NH] = pow2i(max(ev - 14 - 12, -126));  // 2^14 of the weights, 2^12 of the table
   }
   // the parts' rows add up: four heads, lane groups 0 + 1 (a pair's first coordinate) and 2 + 3 (its second); eight,
   // groups 0 + 2 (heads 0 - 3) and 1 + 3 (heads 4 - 7)
@@ -844,7 +846,7 @@ __global__ __launch_bounds__(64 * max_waves(Q8)) void attn_codes(AttnArgs a) {
       const float* st = s_stat + w * S::kStat;
       const float e = __builtin_amdgcn_exp2f(st[h] - m);
       ls = __builtin_fmaf(st[NH + h], e, ls);
-      o = __builtin_fmaf(((const float*)(s_wave0 + w * S::kWave))[h * D + j], e * st[2 * NH], o);
+      o = __builtin_fmaf(((const float*)(s_wave0 + w * S::kWave))[h * D + j], e, o);
     }
     if (a.chunks > 1) {
       a.ws[a.ws_acc + (((uint64_t)kv * a.nqp + h) * a.chunks + c) * D + j] = o;
