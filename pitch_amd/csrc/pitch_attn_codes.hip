@@ -503,10 +503,12 @@ __global__ __launch_bounds__(64 * max_waves(Q8)) void attn_codes(AttnArgs a) {
       bs[h] = kBias ? uniform(s_hs[NH + h]) : 0.f;
     }
   }
+  // The running maxima start at the lowest finite value: a score of minus infinity then weighs nothing, also in a tile,
+  // a wave or a chunk without any other (relative to a maximum of minus infinity it would weigh NaN).
   float M[NH], l[NH];
 #pragma unroll
   for (int h = 0; h < NH; ++h) {
-    M[h] = -__builtin_inff();
+    M[h] = -__FLT_MAX__;
     l[h] = 0.f;
   }
   constexpr int NA = Q8 ? RC : RC / 2;  // accumulators (four heads: a pair's two coordinates on one's rows)

@@ -173,6 +173,50 @@ def test_range_of_weights(q, what, d, nq, tokens):
     _compare(out[0], lse[0], ro, rl, f"{what} d={d} nq={nq} T={tokens}", TOL if score is None else 1e-4)
 
 
+@pytest.mark.parametrize("tokens", [64, 65, 129, 1100, 2113])
+@pytest.mark.parametrize("d,nq", [(128, 4), (64, 8)])
+def test_infinities_and_nan(q, d, nq, tokens):
+    """Two KV heads; the first head's last token, alone in its tile or not, has a key scale of infinity: a score of minus
+    infinity takes no part (the queries come in pairs q and -q: one of each pair has it), plus infinity and a NaN scale
+    give NaN, and an infinite value scale nothing finite. The second head does not notice."""
+    import torch
+    import pitch_amd as P
+    print(d, nq, tokens, flush=True)
+    rng = np.random.default_rng(tokens + d)
+    kc, kp = _packed(rng, 2, tokens, d, 4)
+    vc, vp = _packed(rng, 2, tokens, d, 3)
+    ks, vs = (np.exp(rng.uniform(0.0, 1.0, (2, tokens))).astype(np.float32) for _ in range(2))
+    Q = rng.standard_normal((2, nq // 2, d))
+    Q = np.concatenate([Q, -Q], 1).astype(np.float32)
+    last = O.turbo_decode(kc[0, -1:], np.ones(1), 4, 101)[0]
+    plus = Q[0].astype(np.float64) @ last > 0
+
+    def run(key, value):
+        k, v = ks.copy(), vs.copy()
+        k[0, -1] *= key
+        v[0, -1] *= value
+        dq, dkc, dks, dvc, dvs = _dev(q, Q, kp, k, vp, v)
+        out, lse = torch.empty(2, nq, d, device=q.device), torch.empty(2, nq, device=q.device)
+        q.enqueueAttentionDecode(dq, dkc, dks, dvc, dvs, out, tokens, P.QuantConfig("turboQuant", d, 4, 101),
+                                 P.QuantConfig("turboQuant", d, 3, 202), qPerKv=nq, kvHeads=2, lse=lse)
+        return out.cpu().numpy().astype(np.float64), lse.cpu().numpy().astype(np.float64)
+
+    def reference(h, n):
+        return O.attention_decode(Q[h].astype(np.float64), kc[h, :n], ks[h, :n], vc[h, :n], vs[h, :n], "turboQuant", 4,
+                                  "turboQuant", 3, 1 / math.sqrt(d), 101, 202)
+
+    inf, nan = float("inf"), float("nan")
+    for key, value in ((inf, 1.0), (nan, 1.0), (1.0, inf), (1.0, nan)):
+        out, lse = run(key, value)
+        _compare(out[1], lse[1], *reference(1, tokens), f"head 1 beside {key} {value}")
+        if key == inf:
+            ro, rl = reference(0, tokens - 1)
+            _compare(out[0][~plus], lse[0][~plus], ro[~plus], rl[~plus], "minus infinity")
+            assert np.isnan(out[0][plus]).all()
+        else:
+            assert not np.isfinite(out[0]).any()
+
+
 def test_threads_of_different_lengths(q):
     """Calls of one kernel variant from several threads, each on a stream of its own, with lengths that take four waves
     a workgroup and sixteen (different amounts of LDS): none is refused and each writes what it writes alone."""
