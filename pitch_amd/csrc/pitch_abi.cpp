@@ -576,8 +576,11 @@ uint64_t attention_workspace_floats(uint32_t dim, uint32_t nqp, uint32_t kv_head
   return (uint64_t)kv_heads * nqp * (3 * dim + tokens + chunks * (2 + dim));
 }
 
-// A wave takes one 64-token tile at a time. Up to 16 tiles (key-bias: 4) a KV head is one workgroup, which writes the
-// output itself; longer calls take one workgroup per compute unit, in multiples of eight chunks per KV head where there
+// A wave takes one 64-token tile at a time. Up to 12 tiles (key-bias: 4) a KV head is one workgroup, which writes the
+// output itself: three waves per SIMD, or two rounds of eight waves. A fourth wave or a third round costs more than
+// splitting and the second launch (us per call, one workgroup and split, d = 128, 8 KV heads: 768 tokens, per-channel
+// keys, four queries 11.2 and 11.9, eight 15.7 and 14.9; 832 tokens 12.7 and 11.9, 18.7 and 14.9; 1024 tokens, unequal
+// widths, one query 13.1 and 11.7). Longer calls take one workgroup per compute unit, in multiples of eight chunks per KV head where there
 // are so many (one for each XCD), of at least two tiles (key-bias: one, since a workgroup's cos and sin rows are bound
 // by what one compute unit reads: 2 KV x 6, 2000 tokens 22.5 us with four, 18.1 with one), and at most 128 chunks,
 // which attn_combine merges in two rounds of loads (one KV head, 30000 tokens, per-channel keys: 16.5 us with 235, 13.6 with 118).
@@ -588,7 +591,7 @@ CodesSplit attention_codes_split(uint32_t dim, uint64_t tokens, uint32_t kv_head
   const uint64_t tiles = (tokens + kTileTokens - 1) / kTileTokens;
   const uint64_t fewest = key_bias ? 1 : 2;
   uint64_t chunks = 1;
-  if (tiles > (key_bias ? 4u : kAttnCodesWaves)) {
+  if (tiles > (key_bias ? 4u : kAttnOneTiles)) {
     chunks = cus / kv_heads;
     if (chunks >= 8) chunks = chunks / 8 * 8;
     chunks = std::min<uint64_t>({chunks, (tiles + fewest - 1) / fewest, kAttnMostChunks});

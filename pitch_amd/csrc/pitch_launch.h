@@ -155,6 +155,7 @@ uint64_t attention_workspace_floats(uint32_t dim, uint32_t nqp, uint32_t kv_head
 // head, waves per workgroup. ws_chunk is the chunk length that the call's workspace was sized with.
 constexpr uint32_t kTileTokens = 64;      // tokens a wave takes at a time
 constexpr uint32_t kAttnCodesWaves = 16;  // most waves per workgroup
+constexpr uint32_t kAttnOneTiles = 12;    // most tiles of a KV head that is one workgroup (without the key-bias term)
 constexpr uint32_t kAttnMostChunks = 128;
 struct CodesSplit {
   uint32_t chunk, chunks, waves;

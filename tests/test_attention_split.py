@@ -37,6 +37,17 @@ def test_partials_fit_the_workspace(split, dim, bias, ws_chunk):
                     assert kv * chunks * (2 + dim) <= floats, label
 
 
+@pytest.mark.parametrize("dim", [64, 128])
+def test_one_workgroup_up_to_twelve_tiles(split, dim):
+    """A KV head of up to 12 tiles of 64 tokens (key-bias: 4) is one workgroup; longer ones are split, since a fourth
+    wave per SIMD, or a third round of eight waves, takes longer than the second launch."""
+    for kv in (1, 8, 24):
+        for bias, most in ((0, 768), (1, 256)):
+            assert split(dim, most, kv, bias, 256)[1] == 1
+            chunk, chunks, _, _ = split(dim, most + 1, kv, bias, 256)
+            assert chunks > 1 and chunk <= 128
+
+
 def test_workspace_is_what_the_size_query_says(split):
     lib = _lib.load()
     cfg = _lib.PitchConfigC(0, 128, 4, 1)

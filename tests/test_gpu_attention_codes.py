@@ -38,7 +38,7 @@ def _dev(q, *arrays):
 # unequal widths reach the kernels at every length
 VECTOR = [("turboQuant", 4, 3, 128, 4, 2), ("turboQuant", 2, 4, 64, 1, 3), ("polarQuant", 3, 4, 128, 8, 1),
           ("turboQuant", 3, 2, 64, 5, 2)]
-TOKENS = [1, 63, 64, 65, 1023, 1024, 1025, 1153, 8191, 20001]
+TOKENS = [1, 63, 64, 65, 768, 769, 1023, 1024, 1025, 1153, 8191, 20001]
 
 
 @pytest.mark.parametrize("tokens", TOKENS)
