@@ -365,7 +365,14 @@ int pitch_selftest_reciprocal(uint64_t* mismatches);
  * when there are several), the waves per workgroup and the floats of the workspace that
  * pitch_attention_workspace_size asks for (workspace_chunk 0; otherwise of one sized with chunks of that many tokens). */
 int pitch_selftest_attention_split(uint32_t dim, uint64_t tokens, uint32_t kv_heads, uint32_t key_bias,
-                                   uint32_t compute_units, uint32_t workspace_chunk, uint64_t split[4]);
+                                   uint32_t head_major, uint32_t compute_units, uint32_t workspace_chunk, uint64_t split[4]);
+
+/* Self-test of the choice of kernels for attention over per-vector caches without the key-bias term, without a device; no
+ * counterpart in the reference. Writes 1 if a call of kv_heads heads x tokens with q_per_kv query heads per KV head on a
+ * device of compute_units runs the kernels for codes of 2-4 bits, 0 if it runs the others. head_major is 1 for caches in
+ * which the rows of a KV head's tokens follow each other. */
+int pitch_selftest_attention_route(uint32_t dim, uint64_t tokens, uint32_t kv_heads, uint32_t q_per_kv, uint32_t key_bits,
+                                   uint32_t value_bits, uint32_t head_major, uint32_t compute_units, uint32_t* codes);
 
 #ifdef __cplusplus
 }

@@ -122,7 +122,8 @@ SIGNATURES = {
     "pitch_enqueue_pack_codes": (_int, [_u32, _u32, _vp, _u64, _u64, _vp, _u64, _u64, _u64, _vp]),
     "pitch_enqueue_unpack_codes": (_int, [_u32, _u32, _vp, _u64, _u64, _vp, _u64, _u64, _u64, _vp]),
     "pitch_selftest_reciprocal": (_int, [ctypes.POINTER(_u64)]),
-    "pitch_selftest_attention_split": (_int, [_u32, _u64, _u32, _u32, _u32, _u32, ctypes.POINTER(_u64)]),
+    "pitch_selftest_attention_split": (_int, [_u32, _u64, _u32, _u32, _u32, _u32, _u32, ctypes.POINTER(_u64)]),
+    "pitch_selftest_attention_route": (_int, [_u32, _u64, _u32, _u32, _u32, _u32, _u32, _u32, ctypes.POINTER(_u32)]),
 }
 
 _lock = threading.Lock()

@@ -576,25 +576,91 @@ uint64_t attention_workspace_floats(uint32_t dim, uint32_t nqp, uint32_t kv_head
   return (uint64_t)kv_heads * nqp * (3 * dim + tokens + chunks * (2 + dim));
 }
 
+// Workgroups per KV head of a long call: one per compute unit, a multiple of eight (one for each XCD) where there are so
+// many. In a token-major cache the rows of one token's heads share cache lines, and workgroups go to the XCDs in turn:
+// four chunks per head put the same tokens of all heads on two XCDs, five spread them over all (48 KV, token-major, d = 64,
+// b = 4, four queries, 16000 tokens: 42.6 us with five, 34.2 with four; with six, 40 KV, 34.4, and 33.7 with four, but d =
+// 128 36.7 and 40.6). The key-bias term's cos and sin rows, of one position for all heads, outweigh that (48 KV, d = 128,
+// 16000 tokens: 118 us with five, 141 with four).
+static uint32_t codes_chunks_per_head(uint32_t kv_heads, bool head_major, bool key_bias, uint32_t cus) {
+  const uint32_t per = cus / kv_heads;
+  return per >= 8 ? per / 8 * 8 : per == 5 && !head_major && !key_bias ? 4 : per;
+}
+
+// Whether the 16-bit matrix-core kernels (pitch_attn_codes.hip) take a call of per-vector keys and values without the
+// key-bias term that they can serve; pitch_attention.hip's take the others. Both sides below are us per call in a graph,
+// pitch_attention.hip's kernels first, token-major caches, equal widths unless said otherwise.
+//   * Calls of one workgroup per KV head always: no second launch (8 KV x 4 queries, d = 128, b = 4, 300 tokens: 11.9
+//     and 10.0). With equal widths attn_chunk has no second scores launch either, so only up to 512 tokens.
+//   * Their fixed cost is the table, 64 KB per workgroup at four bits. With equal widths it pays above 32768 tokens over
+//     all KV heads at d = 128 and 131072 at d = 64 (b = 4: d = 128, 8 KV x 4, 4096 tokens 12.2 and 12.8, 6000 tokens
+//     15.6 and 12.7; 2 KV x 4, 16384 tokens 13.6 and 14.6; 1 KV x 1, 65536 tokens 20.0 and 13.6; d = 64, 12 KV x 1, 8192
+//     tokens 10.5 and 11.5, 16000 tokens 18.9 and 15.0). One query per KV head leaves attn_chunk the least to do: at
+//     d = 128 and four bits it serves up to 65536 tokens as long as a head has at most 4096 (12 KV, 4000 tokens 11.0 and
+//     11.7; 64 KV, 1000 tokens 11.3 and 12.7; 8 KV, 6000 tokens 12.0 and 11.7), and with unequal widths, one of four
+//     bits, up to 32768 (2 KV, 16000 tokens, PolarQuant 4/3 12.9 and 13.8, 12 KV, 2000 tokens 11.7 and 12.3; 8 KV, 8000
+//     tokens 4/2 15.3 and 12.5; 3/2, 8 KV, 1000 tokens 11.5 and 10.7).
+//   * One workgroup per compute unit only fills the device if the KV heads share its compute units out, and the rows of
+//     one token's heads are read by few XCDs only if a head's chunks are a multiple or a divisor of eight. Of five to
+//     seven chunks per head, calls of few queries stay with attn_chunk (b = 4, 40 KV: one query, d = 64, 16000 tokens
+//     28.2 and 34.1, d = 128, 2000 tokens 13.3 and 14.5, but 16000 tokens 41.1 and 36.3; four queries, d = 64, 8000
+//     tokens 20.9 and 22.6; eight 28.8 and 26.7). With idle compute units one query loses at d = 64 (20 KV, 32000 tokens
+//     27.7 and 30.5; 16 KV, which has none idle, 24.5 and 20.2) and at two bits (d = 128, 20 KV, 8000 tokens 14.1 and
+//     16.1); with up to a sixteenth as many heads as compute units only in long calls (12 KV, d = 64, 32000 tokens 26.7
+//     and 19.5, 65536 tokens 27.9 and 29.6).
+//   * In head-major caches attn_chunk reads each head in one piece, which one query feels most, at two bits and if there
+//     are enough heads for its chunks to be short (12 KV, d = 64,
+//     16000 tokens 10.7 and 12.4; 48 KV, d = 128, 2000 tokens 11.2 and 11.7, 8000 tokens 20.2 and 18.8; b = 4: 8 KV, d =
+//     128, 8000 tokens 11.0 and 11.7, 16000 tokens 16.0 and 12.8; 12 KV, d = 64, 16000 tokens 12.3 and 13.0, 32000 tokens
+//     17.5 and 16.6); idle compute units only matter at two bits (20 KV, d = 64, 16000 tokens 14.8 and 16.5; b = 4 17.1
+//     and 16.7).
+// Per-channel keys and the key-bias term take three or four launches in pitch_attention.hip and are faster in the 16-bit
+// kernels at every size (8 KV x 4, 300 tokens, per-channel: 14.2 and 9.7; 4096: 14.4 and 11.5).
+bool attention_codes_pays(uint32_t dim, uint64_t tokens, uint32_t kv_heads, uint32_t padded_queries, uint32_t kbits,
+                          uint32_t vbits, bool head_major, uint32_t cus) {
+  const bool wide = dim == 128, equal = kbits == vbits, single = padded_queries == 1;
+  const uint32_t bits = std::max(kbits, vbits);
+  if (tokens <= (equal ? 512u : kAttnOneTiles * kTileTokens)) return true;
+  uint64_t least = 0;
+  if (equal && single && head_major && kv_heads >= cus / 32)
+    least = !wide ? (bits == 2 ? 245760 : 196608) : bits == 2 ? 98304 : tokens <= 8192 ? 65536 : 32768;
+  else if (equal) least = !wide ? 131072 : single && bits == 4 && tokens <= 4096 ? 65536 : 32768;
+  else if (single && bits == 4) least = 32768;
+  if (tokens <= least / kv_heads) return false;
+  const uint32_t per = cus / kv_heads;  // workgroups that a KV head can have
+  if (!head_major && per >= 5 && per <= 7) {
+    if (single && equal) return wide && bits == 4 && per > 5 && tokens > 4096;
+    if (single) return per > 5 && (wide ? bits == 4 && tokens > 2048 : bits < 4 && (per == 6 || tokens <= 1024));
+    if (!wide && equal && padded_queries <= 4) return bits < 4 && per == 6;
+    if (!wide && padded_queries == 2) return bits < 4 || per != 7;
+  }
+  if (single && equal && kv_heads > cus / 32) {
+    const uint32_t busy = kv_heads * codes_chunks_per_head(kv_heads, head_major, false, cus);
+    if (head_major) return bits > 2 || 4 * busy > 3 * cus;
+    if (kv_heads > cus / 16 || tokens > 655360 / kv_heads)
+      return wide ? bits > 2 || 4 * busy > 3 * cus : 16 * busy >= 15 * cus;
+  }
+  return true;
+}
+
 // A wave takes one 64-token tile at a time. Up to 12 tiles (key-bias: 4) a KV head is one workgroup, which writes the
 // output itself: three waves per SIMD, or two rounds of eight waves. A fourth wave or a third round costs more than
 // splitting and the second launch (us per call, one workgroup and split, d = 128, 8 KV heads: 768 tokens, per-channel
 // keys, four queries 11.2 and 11.9, eight 15.7 and 14.9; 832 tokens 12.7 and 11.9, 18.7 and 14.9; 1024 tokens, unequal
-// widths, one query 13.1 and 11.7). Longer calls take one workgroup per compute unit, in multiples of eight chunks per KV head where there
-// are so many (one for each XCD), of at least two tiles (key-bias: one, since a workgroup's cos and sin rows are bound
-// by what one compute unit reads: 2 KV x 6, 2000 tokens 22.5 us with four, 18.1 with one), and at most 128 chunks,
-// which attn_combine merges in two rounds of loads (one KV head, 30000 tokens, per-channel keys: 16.5 us with 235, 13.6 with 118).
+// widths, one query 13.1 and 11.7). Longer calls take one workgroup per compute unit (codes_chunks_per_head) of at least
+// two tiles (key-bias: one, since a workgroup's cos and sin rows are bound by what one compute unit reads: 2 KV x 6, 2000
+// tokens 22.5 us with four, 18.1 with one), and at most 128 chunks, which attn_combine merges in two rounds of loads (one KV head, 30000 tokens, per-channel keys: 16.5 us with
+// 235, 13.6 with 118).
 // The partials of all chunks fit the caller's workspace by construction: it holds 3 d + tokens floats per padded query
 // and 2 + d for every chunk of ws_chunk tokens (attention_workspace_floats).
-CodesSplit attention_codes_split(uint32_t dim, uint64_t tokens, uint32_t kv_heads, bool key_bias, uint32_t cus,
-                                 uint32_t ws_chunk) {
+CodesSplit attention_codes_split(uint32_t dim, uint64_t tokens, uint32_t kv_heads, bool key_bias, bool head_major,
+                                 uint32_t cus, uint32_t ws_chunk) {
   const uint64_t tiles = (tokens + kTileTokens - 1) / kTileTokens;
   const uint64_t fewest = key_bias ? 1 : 2;
   uint64_t chunks = 1;
   if (tiles > (key_bias ? 4u : kAttnOneTiles)) {
-    chunks = cus / kv_heads;
-    if (chunks >= 8) chunks = chunks / 8 * 8;
-    chunks = std::min<uint64_t>({chunks, (tiles + fewest - 1) / fewest, kAttnMostChunks});
+    chunks = std::min<uint64_t>(
+        {codes_chunks_per_head(kv_heads, head_major, key_bias, cus), (tiles + fewest - 1) / fewest, kAttnMostChunks});
     chunks = std::max<uint64_t>(chunks, (tiles >> 24) + 1);  // a chunk's tokens are counted in 32 bits
     chunks = std::min<uint64_t>(chunks, attention_workspace_floats(dim, 1, 1, tokens, ws_chunk) / (2 + dim));
   }
@@ -1167,17 +1233,27 @@ int pitch_selftest_reciprocal(uint64_t* mismatches) {
 }
 
 int pitch_selftest_attention_split(uint32_t dim, uint64_t tokens, uint32_t kv_heads, uint32_t key_bias,
-                                   uint32_t compute_units, uint32_t workspace_chunk, uint64_t split[4]) {
+                                   uint32_t head_major, uint32_t compute_units, uint32_t workspace_chunk, uint64_t split[4]) {
   if (!split) return fail(PITCH_ERR_INVALID_INPUT, "split is null");
   if (dim == 0 || tokens == 0 || kv_heads == 0)
     return fail(PITCH_ERR_INVALID_INPUT, "dimension, tokens and KV heads must be at least 1");
   const uint32_t chunk = workspace_chunk ? workspace_chunk : pitch::attention_chunk_tokens(tokens, kv_heads);
   const pitch::CodesSplit x =
-      pitch::attention_codes_split(dim, tokens, kv_heads, key_bias != 0, compute_units, chunk);
+      pitch::attention_codes_split(dim, tokens, kv_heads, key_bias != 0, head_major != 0, compute_units, chunk);
   split[0] = x.chunk;
   split[1] = x.chunks;
   split[2] = x.waves;
   split[3] = pitch::attention_workspace_floats(dim, 1, kv_heads, tokens, chunk);
+  return ok();
+}
+
+int pitch_selftest_attention_route(uint32_t dim, uint64_t tokens, uint32_t kv_heads, uint32_t q_per_kv, uint32_t key_bits,
+                                   uint32_t value_bits, uint32_t head_major, uint32_t compute_units, uint32_t* codes) {
+  if (!codes) return fail(PITCH_ERR_INVALID_INPUT, "codes is null");
+  if (tokens == 0 || kv_heads == 0 || q_per_kv == 0)
+    return fail(PITCH_ERR_INVALID_INPUT, "tokens, KV heads and queries must be at least 1");
+  *codes = pitch::attention_codes_pays(dim, tokens, kv_heads, padded_queries(q_per_kv), key_bits, value_bits,
+                                       head_major != 0, compute_units);
   return ok();
 }
 

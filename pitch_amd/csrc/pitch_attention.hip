@@ -1022,28 +1022,23 @@ hipError_t launch_nq(const AttnArgs& a, hipStream_t s) {
 // They take key and value widths of 2, 3 and 4 bits, both codecs of one kind, and caches of which 64 token rows span
 // less than 2^31 bytes (a tile's rows are addressed with 32-bit offsets). Wider codes, whose tables would not fit the
 // LDS in 32 copies, keys and values of different per-vector methods, and enormous strides stay with this file's kernels.
-// So do the short calls of per-vector keys and values of equal width without the key-bias term, which attn_chunk
-// serves: the kernels' fixed cost (64 KB of table per workgroup) only pays from 32768 tokens over all KV heads at
-// d = 128 and 131072 at d = 64. Both sides there, us per call in a graph, b = 4: d = 128, 8 KV x 4 queries, 4096
-// tokens 12.2 here, 12.8 there; 6000 tokens 15.6 and 12.7; 2 KV x 4, 16384 tokens 13.6 and 14.6; 1 KV x 1, 65536
-// tokens 20.0 and 13.6; d = 64, 12 KV x 1, 8192 tokens 10.5 and 11.5; 16000 tokens 18.9 and 15.0. Up to 512 tokens
-// those calls go there too, since one workgroup then holds a KV head and there is no second launch (300 tokens, 8 KV x
-// 4: 11.9 and 10.0). Per-channel keys, the key-bias term and unequal widths take three or four launches here and are
-// faster there at every size (8 KV x 4, 300 tokens, per-channel: 14.2 and 9.7; 4096: 14.4 and 11.5).
+// So do the calls of per-vector keys and values without the key-bias term that these are faster for
+// (attention_codes_pays).
 int codes_kind(const AttnArgs& a) {
   if (a.kbits > 4 || a.vbits > 4) return -1;
   if (a.token_stride > (1ull << 31) / (kTileTokens * PITCH_DIM)) return -1;
   if (a.k_ranges) return a.vpolar ? kAttnKindChanPolar : kAttnKindChanTurbo;
   if ((a.kpolar != 0) != (a.vpolar != 0)) return -1;
   if (a.kb_cos) return a.kpolar ? kAttnKindPolarBias : kAttnKindTurboBias;
-  constexpr uint64_t kShort = PITCH_DIM == 128 ? 32768 : 131072;
-  if (a.kbits == a.vbits && a.tokens > 512 && a.tokens <= kShort / a.kv_heads) return -1;
+  if (!attention_codes_pays(a.dim, a.tokens, a.kv_heads, a.nqp, a.kbits, a.vbits, a.token_stride == 1,
+                            (uint32_t)device_cu_count()))
+    return -1;
   return a.kpolar ? kAttnKindPolar : kAttnKindTurbo;
 }
 
 // Sets a call's work split (attention_codes_split) and workspace regions, returns the waves per workgroup.
 uint32_t codes_split(AttnArgs& a) {
-  const CodesSplit x = attention_codes_split(a.dim, a.tokens, a.kv_heads, a.kb_cos != nullptr,
+  const CodesSplit x = attention_codes_split(a.dim, a.tokens, a.kv_heads, a.kb_cos != nullptr, a.token_stride == 1,
                                              (uint32_t)device_cu_count(), a.chunk);
   a.chunk = x.chunk;
   a.chunks = x.chunks;

@@ -160,8 +160,10 @@ constexpr uint32_t kAttnMostChunks = 128;
 struct CodesSplit {
   uint32_t chunk, chunks, waves;
 };
-CodesSplit attention_codes_split(uint32_t dim, uint64_t tokens, uint32_t kv_heads, bool key_bias, uint32_t cus,
-                                 uint32_t ws_chunk);
+CodesSplit attention_codes_split(uint32_t dim, uint64_t tokens, uint32_t kv_heads, bool key_bias, bool head_major,
+                                 uint32_t cus, uint32_t ws_chunk);
+bool attention_codes_pays(uint32_t dim, uint64_t tokens, uint32_t kv_heads, uint32_t padded_queries, uint32_t kbits,
+                          uint32_t vbits, bool head_major, uint32_t cus);
 hipError_t launch_attention_d64(const AttnArgs& a, hipStream_t s);
 hipError_t launch_attention_d128(const AttnArgs& a, hipStream_t s);
 

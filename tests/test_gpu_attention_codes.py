@@ -35,9 +35,10 @@ def _dev(q, *arrays):
     return [torch.from_numpy(np.ascontiguousarray(a)).to(q.device) for a in arrays]
 
 
-# unequal widths reach the kernels at every length
+# unequal widths reach the kernels at every length, with one query only those below four bits (a call of 2 and 4 bits from
+# 769 tokens to 32768 over all heads runs pitch_attention.hip's)
 VECTOR = [("turboQuant", 4, 3, 128, 4, 2), ("turboQuant", 2, 4, 64, 1, 3), ("polarQuant", 3, 4, 128, 8, 1),
-          ("turboQuant", 3, 2, 64, 5, 2)]
+          ("turboQuant", 3, 2, 64, 5, 2), ("turboQuant", 2, 3, 64, 1, 3)]
 TOKENS = [1, 63, 64, 65, 768, 769, 1023, 1024, 1025, 1153, 8191, 20001]
 
 
