@@ -649,8 +649,8 @@ bool attention_codes_pays(uint32_t dim, uint64_t tokens, uint32_t kv_heads, uint
 // keys, four queries 11.2 and 11.9, eight 15.7 and 14.9; 832 tokens 12.7 and 11.9, 18.7 and 14.9; 1024 tokens, unequal
 // widths, one query 13.1 and 11.7). Longer calls take one workgroup per compute unit (codes_chunks_per_head) of at least
 // two tiles (key-bias: one, since a workgroup's cos and sin rows are bound by what one compute unit reads: 2 KV x 6, 2000
-// tokens 22.5 us with four, 18.1 with one), and at most 128 chunks, which attn_combine merges in two rounds of loads (one KV head, 30000 tokens, per-channel keys: 16.5 us with
-// 235, 13.6 with 118).
+// tokens 22.5 us with four, 18.1 with one), and at most 128 chunks, which attn_combine merges in two rounds of loads (one
+// KV head, 30000 tokens, per-channel keys: 16.5 us with 235, 13.6 with 118).
 // The partials of all chunks fit the caller's workspace by construction: it holds 3 d + tokens floats per padded query
 // and 2 + d for every chunk of ws_chunk tokens (attention_workspace_floats).
 CodesSplit attention_codes_split(uint32_t dim, uint64_t tokens, uint32_t kv_heads, bool key_bias, bool head_major,

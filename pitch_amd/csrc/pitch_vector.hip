@@ -2387,16 +2387,21 @@ constexpr EncKind enc_kind() {
   return EncKind::kTeam;
 }
 // Whether a call of so many vectors runs the LDS-transposed encoder where enc_kind names it; the others run the team
-// encoder, with the same bytes. 16-bit TurboQuant takes it from 2^23 coordinates: below two of its resident rounds
-// (2 waves per SIMD against the team encoder's 4) its fixed cost loses. us per call, team and transposed, d = 256,
-// bfloat16: 64 vectors, b = 2: 4.4 and 5.2; 16744, b = 4: 7.7 and 9.3; 40000, b = 8: 13.8 and 13.5; 131072, b = 3: 41.0
-// and 31.8 (d = 512 and 1024 alike). PolarQuant gains at every size (the same four: 6.7 and 5.8, 12.9 and 11.0, 23.3
-// and 18.4, 68.8 and 35.1), float32 was measured faster before.
-template <int D, bool POLAR, int IO>
-constexpr bool lt_by_size() { return IO != 0 && !POLAR; }
-template <int D, bool POLAR, int IO>
+// encoder, with the same bytes. Both sides below are us per call, team and transposed, d = 256, bfloat16 (float16, d = 512
+// and 1024 alike). 16-bit TurboQuant takes it from 2^23 coordinates: below two of its resident rounds (2 waves per SIMD
+// against the team encoder's 4) its fixed cost loses (64 vectors, b = 2: 4.4 and 5.2; 16744, b = 4: 7.7 and 9.3; 40000, b =
+// 8: 13.8 and 13.5; 131072, b = 3: 41.0 and 31.8). PolarQuant of 2 - 5 bits gains at every size (64 vectors, b = 2: 6.7
+// and 5.8, b = 5: 6.6 and 6.3; 4096, b = 5: 8.7 and 7.3; 131072, b = 3: 68.8 and 35.1). Its octant table grows with 2^b, so
+// with 6 - 8 bits only calls of next to no work, 2^12 coordinates, and from 2^22 (b = 8: above it) gain (b = 8: 1 vector
+// 5.3 and 4.9, 16 5.9 and 5.8, 32 6.2 and 6.6, 512 8.0 and 8.5, 16384 11.6 and 11.8, 24576 14.8 and 13.5; d = 512, 512
+// vectors 8.4 and 9.2; b = 6, d = 512, 256 vectors 7.6 and 8.4, 8192 12.1 and 11.2). float32 was measured faster at every
+// size.
+template <int B, bool POLAR, int IO>
+constexpr bool lt_by_size() { return IO != 0 && (!POLAR || B >= 6); }
+template <int D, int B, bool POLAR, int IO>
 bool lt_pays(uint64_t vectors) {
-  return !lt_by_size<D, POLAR, IO>() || vectors >= (1u << 23) / D;
+  if constexpr (!lt_by_size<B, POLAR, IO>()) return true;
+  return POLAR ? vectors <= (1u << 12) / D || vectors >= (1u << 22) / D + (B == 8) : vectors >= (1u << 23) / D;
 }
 // Vectors a workgroup of that encoder (without key bias) takes per round.
 template <int D, bool POLAR, int IO>
@@ -2442,7 +2447,7 @@ hipError_t launch_one(bool encode, const VecArgs& args, hipStream_t s) {
     }
   }
   if constexpr (kEnc == EncKind::kTransposed) {
-    if (encode && lt_pays<D, POLAR, IO>(a.count)) {
+    if (encode && lt_pays<D, B, POLAR, IO>(a.count)) {
       using L = Lt<D, POLAR>;
       fill_lt_flips<D>(a.seed, a.lane_flips);
       const uint64_t need = (a.count + L::WAVES * L::V - 1) / (L::WAVES * L::V);
@@ -2469,7 +2474,7 @@ hipError_t launch_one(bool encode, const VecArgs& args, hipStream_t s) {
   fill_lane_flips<D>(a.seed, a.lane_flips);
   const uint64_t need = (a.count + G::VPB - 1) / G::VPB;
   if (encode) {
-    if constexpr (kEnc == EncKind::kTeam || (kEnc == EncKind::kTransposed && lt_by_size<D, POLAR, IO>())) {
+    if constexpr (kEnc == EncKind::kTeam || (kEnc == EncKind::kTransposed && lt_by_size<B, POLAR, IO>())) {
       const void* k = (const void*)&vec_encode<D, B, POLAR, IO, KBIAS>;
       const uint64_t grid = persistent_grid(k, need);
       hipLaunchKernelGGL((vec_encode<D, B, POLAR, IO, KBIAS>), dim3((uint32_t)grid), dim3(kBlock), 0, s, a);
@@ -2580,7 +2585,7 @@ hipError_t launch_batch(VecBatchArgs a, hipStream_t s) {
   uint64_t total = 0;
   for (uint32_t j = 0; j < a.items; ++j) total += a.count[j];
   if constexpr (k == EncKind::kTransposed) {
-    if (lt_pays<D, POLAR, PITCH_IO>(total)) {
+    if (lt_pays<D, B, POLAR, PITCH_IO>(total)) {
       const void* kp = (const void*)&vec_encode_lt_batch<D, B, POLAR, PITCH_IO>;
       bool fair = false;
       const dim3 grid(assign_blocks(a, vpb, [&](uint64_t t) {
@@ -2615,7 +2620,7 @@ hipError_t launch_batch(VecBatchArgs a, hipStream_t s) {
     }));
     a.common.fair = fair ? 1u : 0u;
     hipLaunchKernelGGL((tq_encode_lpv_batch<D, B, PITCH_IO>), grid, dim3(64), 0, s, a);
-  } else if constexpr (k == EncKind::kTeam || lt_by_size<D, POLAR, PITCH_IO>()) {
+  } else if constexpr (k == EncKind::kTeam || lt_by_size<B, POLAR, PITCH_IO>()) {
     const void* kp = (const void*)&vec_encode_batch<D, B, POLAR, PITCH_IO>;
     const dim3 grid(assign_blocks(a, Geom<D>::VPB, [&](uint64_t t) { return persistent_grid(kp, t); }));
     fill_lane_flips<D>(a.common.seed, a.common.lane_flips);
