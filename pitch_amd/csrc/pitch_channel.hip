@@ -734,10 +734,30 @@ bool wave_decodes_32(const ChanArgs& a) {
   return a.group == 32u && (IO != 0 || a.count <= 16384u);
 }
 
+// Whether an encode runs the wave encoder: groups of up to 64 rows always, those of 65 to 128 if 128 rows' work in 32
+// channels at a time is worth it. Whole slabs are, and so is a dimension above 64. A partial slab keeps lanes idle and,
+// with widths other than 2, 4 and 8, packs its rows code by code; chan_encode4, one workgroup for all channels of a group,
+// is faster then, more so for long groups, until it fills the device. us per call, chan_encode4 and the wave encoder,
+// float32, 16000 tokens, groups of 65 and of 128: d = 64, b = 4 6.2 and 4.9, 7.7 and 5.1; d = 68, b = 3 8.5 and 6.8, 14.5
+// and 7.3; d = 24, b = 3 6.2 and 10.4, 8.3 and 12.2, b = 4 6.0 and 7.5, 7.6 and 8.8; d = 44, b = 3 7.6 and 8.8, 10.3 and
+// 10.4, b = 4 6.7 and 7.1, 8.8 and 8.1; d = 60, b = 5 8.2 and 11.0, 11.8 and 15.0, 64000 tokens 15.8 and 13.0, 14.2 and
+// 15.5.
+template <int B>
+bool wave_encodes(const ChanArgs& a) {
+  if (a.group > (uint32_t)kGroupMaxW) return false;
+  if (a.group <= 64u || a.dim % 32u == 0u || a.dim > 64u) return true;
+  constexpr bool kBytes = B == 2 || B == 4 || B == 8;
+  const bool shorter = a.group < 96u, many = a.count > 32768u;
+  if (a.dim < 32u)
+    return a.dim <= (kBytes ? 12u : 8u) || (many && shorter) || (kBytes && a.dim == 16u && (many || a.group < 128u));
+  if (a.dim <= 52u) return kBytes || a.dim <= 40u || !shorter || many;
+  return many && (kBytes || shorter);
+}
+
 template <int B, int IO>
 hipError_t launch_b(bool encode, const ChanArgs& a, hipStream_t s) {
   const bool vec4 = (a.dim & 3u) == 0u;
-  if (encode && vec4 && a.group <= (uint32_t)kGroupMaxW) {
+  if (encode && vec4 && wave_encodes<B>(a)) {
     const uint64_t groups = ((uint64_t)a.count + a.group - 1) / a.group;
     // 32-channel slabs double the work items and halve each lane's registers, which balances float32 calls
     // with few (group, 64-channel) items over the resident waves (+5-10 % at 4096-8192 items); long calls keep

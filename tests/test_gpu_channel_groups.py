@@ -35,3 +35,23 @@ def test_bits(q, dim, bits, group, io):
     q.enqueuePerChannelDecode(c, r, out, tokens, cfg)
     want = O.to_io_bits(O.channel_decode(codes, ranges, bits, group), io)
     assert np.array_equal(out.cpu().view(torch.int32 if io == "float32" else torch.int16).numpy().view(want.dtype), want)
+
+
+@pytest.mark.parametrize("io", ["float32", "bfloat16"])
+@pytest.mark.parametrize("tokens", [130, 1000, 32768, 32769])
+@pytest.mark.parametrize("group", [65, 96, 128])
+@pytest.mark.parametrize("dim,bits", [(12, 2), (16, 8), (12, 5), (28, 4), (36, 3), (44, 3), (52, 2), (56, 6), (60, 5), (60, 8)])
+def test_partial_slabs(q, dim, bits, group, tokens, io):
+    """Groups of 65 to 128 rows whose channels do not fill slabs of 32: both encoders at both sides of their rule."""
+    import torch
+    print(f"d={dim} b={bits} G={group} {io} {tokens}", flush=True)
+    rng = np.random.default_rng(dim * 1000 + group + tokens)
+    x = rng.standard_normal((tokens, dim)).astype(np.float32)
+    t = torch.from_numpy(x).to(getattr(torch, io))
+    codes, ranges = O.channel_encode(t.float().numpy(), bits, group)
+    cfg = q.channelConfig(dim, bits, group)
+    c = torch.zeros(tokens * cfg.codeStride, dtype=torch.uint8, device=q.device)
+    r = torch.zeros(ranges.size, dtype=torch.int16, device=q.device)
+    q.enqueuePerChannelEncode(t.to(q.device), c, r, tokens, cfg)
+    assert c.cpu().numpy().tobytes() == O.pack_codes(codes, bits)
+    assert np.array_equal(r.cpu().numpy().view(np.uint16), ranges.reshape(-1).view(np.uint16))
