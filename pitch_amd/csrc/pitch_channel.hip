@@ -724,14 +724,16 @@ __global__ __launch_bounds__(kBlock) void chan_decode1(ChanArgs p) {
   }
 }
 
-// Whether a decode of 32-token groups runs the wave decoder in chunks of 32: every 16-bit call, and float32 calls of few
-// tokens. us per call, chan_decode4 and the wave decoder, b = 4: bfloat16, 8 heads x 32768 tokens, d = 64 15.0 and
-// 9.8, d = 80 19.1 and 17.4, d = 128 21.5 and 20.1; float32, 2048 tokens, d = 64 3.6 and 2.7, d = 128 3.4 and 2.7, but
-// 8 x 32768 tokens at d = 80 20.3 and 26.8, d = 128 26.3 and 30.7 (a lane's range set-up serves four rows only).
+// Whether a decode of 32-token groups runs the wave decoder in chunks of 32: 16-bit calls of more than one group (or of
+// more than 80 channels), and float32 calls of few tokens. us per call, chan_decode4 and the wave decoder, b = 4: bfloat16,
+// 8 heads x 32768 tokens, d = 64 15.0 and 9.8, d = 80 19.1 and 17.4, d = 128 21.5 and 20.1; 64 tokens, d = 64 3.3 and 2.8,
+// d = 80 3.5 and 3.1; one group, d = 64 2.5 and 2.7, d = 80 2.7 and 2.8, d = 128 3.0 and 2.8. float32, d = 64 and d = 128:
+// 2048 tokens 3.6 and 2.7, 3.4 and 2.7; 16384 4.0 and 3.2, 4.0 and 3.4; 65536 5.4 and 4.5, 7.4 and 6.9; but 8 x 32768 at
+// d = 80 20.3 and 26.8, at d = 128 26.3 and 30.7 (a lane's range set-up serves four rows only).
 // Other multiples of 32 keep chan_decode4 (groups of 96, d = 96, bfloat16, 4 x 20000 tokens: 18.2 and 22.7).
 template <int IO>
 bool wave_decodes_32(const ChanArgs& a) {
-  return a.group == 32u && (IO != 0 || a.count <= 16384u);
+  return a.group == 32u && (IO != 0 ? a.count > 32u || a.dim > 80u : a.count <= 16384u);
 }
 
 // Whether an encode runs the wave encoder: groups of up to 64 rows always, those of 65 to 128 if 128 rows' work in 32

@@ -55,3 +55,21 @@ def test_partial_slabs(q, dim, bits, group, tokens, io):
     q.enqueuePerChannelEncode(t.to(q.device), c, r, tokens, cfg)
     assert c.cpu().numpy().tobytes() == O.pack_codes(codes, bits)
     assert np.array_equal(r.cpu().numpy().view(np.uint16), ranges.reshape(-1).view(np.uint16))
+
+
+@pytest.mark.parametrize("io", ["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize("tokens", [1, 31, 32, 33, 64])
+@pytest.mark.parametrize("dim,bits", [(64, 4), (80, 3), (84, 2), (128, 8)])
+def test_decode_of_few_groups_of_32(q, dim, bits, tokens, io):
+    """One group of 32 tokens, whole or not, and two: the decoders at both sides of their rule."""
+    import torch
+    print(f"d={dim} b={bits} {io} {tokens}", flush=True)
+    rng = np.random.default_rng(dim + tokens)
+    codes, ranges = O.channel_encode(rng.standard_normal((tokens, dim)).astype(np.float32), bits, 32)
+    cfg = q.channelConfig(dim, bits, 32)
+    c = torch.from_numpy(np.frombuffer(O.pack_codes(codes, bits), np.uint8).copy()).to(q.device)
+    r = torch.from_numpy(ranges.reshape(-1).view(np.int16).copy()).to(q.device)
+    out = torch.zeros((tokens, dim), dtype=getattr(torch, io), device=q.device)
+    q.enqueuePerChannelDecode(c, r, out, tokens, cfg)
+    want = O.to_io_bits(O.channel_decode(codes, ranges, bits, 32), io)
+    assert np.array_equal(out.cpu().view(torch.int32 if io == "float32" else torch.int16).numpy().view(want.dtype), want)
