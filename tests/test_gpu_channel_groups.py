@@ -73,3 +73,19 @@ def test_decode_of_few_groups_of_32(q, dim, bits, tokens, io):
     q.enqueuePerChannelDecode(c, r, out, tokens, cfg)
     want = O.to_io_bits(O.channel_decode(codes, ranges, bits, 32), io)
     assert np.array_equal(out.cpu().view(torch.int32 if io == "float32" else torch.int16).numpy().view(want.dtype), want)
+
+
+@pytest.mark.parametrize("tokens", [4095, 4096, 4097, 5000])
+@pytest.mark.parametrize("dim,bits,group", [(64, 3, 32), (80, 5, 16), (96, 6, 17), (128, 7, 32)])
+def test_rows_of_small_groups(q, dim, bits, group, tokens):
+    """float32 groups of up to 32 rows, widths that are packed code by code: 64 and 32 rows per wave."""
+    import torch
+    print(f"d={dim} b={bits} G={group} {tokens}", flush=True)
+    x = np.random.default_rng(dim + tokens).standard_normal((tokens, dim)).astype(np.float32)
+    codes, ranges = O.channel_encode(x, bits, group)
+    cfg = q.channelConfig(dim, bits, group)
+    c = torch.zeros(tokens * cfg.codeStride, dtype=torch.uint8, device=q.device)
+    r = torch.zeros(ranges.size, dtype=torch.int16, device=q.device)
+    q.enqueuePerChannelEncode(torch.from_numpy(x).to(q.device), c, r, tokens, cfg)
+    assert c.cpu().numpy().tobytes() == O.pack_codes(codes, bits)
+    assert np.array_equal(r.cpu().numpy().view(np.uint16), ranges.reshape(-1).view(np.uint16))
