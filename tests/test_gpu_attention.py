@@ -11,10 +11,12 @@ relative, so those cases use 1e-4.
 
 Cases cover every kernel instantiation family: d = 64 and 128; key and value bit widths 2..8 (pair tables for
 b <= 5, two-level tables above), both methods on either side, different seeds for K and V, query heads per KV
-head 1..8 (padded to 1, 2, 4, 8), one to three KV heads, token counts from 1 to 70,000 (one to many chunks,
-chunk lengths 256 / 512 / 1024), head-major and token-major caches, and end-to-end encoded caches. Equal key
+head 1..8 (padded to 1, 2, 4, 8), one to four KV heads, token counts from 1 to 140,000 (one to many chunks,
+chunk lengths 128 / 256 / 512 / 1024), head-major and token-major caches, and end-to-end encoded caches. Equal key
 and value widths run the fused scores-and-values kernel (attn_chunk), including equal widths with different
-methods, where it rebuilds its table between the phases; unequal widths run the separate kernels.
+methods, where it rebuilds its table between the phases; unequal widths run the separate kernels. Most calls of both
+widths in 2..4 and one method, of per-channel keys and of the key-bias term run the 16-bit matrix-core kernels instead
+(tests/test_gpu_attention_codes.py covers those); cases above four bits keep the others in every form.
 """
 import math
 
@@ -71,12 +73,18 @@ CASES = [
     ("turboQuant", "turboQuant", 8, 2, 128, 4, 2, 2000),   # the reference's mixed (key, value) bits
     ("turboQuant", "turboQuant", 4, 2, 64, 4, 1, 1),
     ("turboQuant", "turboQuant", 4, 4, 128, 4, 1, 7),
-    ("turboQuant", "turboQuant", 4, 4, 128, 4, 2, 70000),  # many chunks, 512-token chunks
-    ("turboQuant", "turboQuant", 3, 3, 64, 2, 3, 140000),  # 1024-token chunks
-    # unequal widths with 4 or 8 padded query heads: the separate scores and values kernels in matrix-core form
+    ("turboQuant", "turboQuant", 4, 4, 128, 4, 2, 70000),  # (these two: the 16-bit matrix-core kernels)
+    ("turboQuant", "turboQuant", 3, 3, 64, 2, 3, 140000),
+    ("turboQuant", "turboQuant", 8, 8, 128, 4, 2, 70000),  # 256-token chunks
+    ("turboQuant", "turboQuant", 5, 5, 64, 2, 3, 140000),  # 512-token chunks
+    ("polarQuant", "polarQuant", 5, 5, 128, 8, 4, 140000),  # 1024-token chunks
+    # unequal widths with 4 or 8 padded query heads (above four bits, or of two methods): the separate scores and values
+    # kernels in matrix-core form
     ("turboQuant", "turboQuant", 4, 2, 64, 8, 2, 3000),
     ("polarQuant", "turboQuant", 3, 4, 128, 7, 1, 1500),
     ("turboQuant", "polarQuant", 2, 3, 64, 3, 2, 900),
+    ("turboQuant", "turboQuant", 5, 2, 64, 8, 2, 3000),
+    ("turboQuant", "turboQuant", 8, 5, 128, 4, 2, 70000),
 ]
 
 
@@ -223,6 +231,10 @@ CHANNEL_CASES = [
     (4, 3, 128, 64, 8, 1, 65),
     (5, 4, 64, 128, 2, 2, 1),
     (4, 4, 128, 64, 4, 1, 70000),
+    (8, 5, 128, 64, 4, 2, 3000),
+    (5, 8, 128, 128, 8, 1, 5000),
+    (6, 4, 128, 64, 1, 2, 5000),
+    (8, 4, 64, 64, 8, 1, 70000),
 ]
 
 
@@ -279,6 +291,8 @@ KEY_BIAS_CASES = [
     ("turboQuant", "polarQuant", 3, 4, 64, 1, 2, 777, 5),
     ("turboQuant", "turboQuant", 2, 2, 64, 8, 1, 70000, 100),
     ("polarQuant", "polarQuant", 5, 3, 128, 5, 1, 300, 0),
+    ("turboQuant", "turboQuant", 5, 5, 64, 8, 1, 20000, 100),
+    ("polarQuant", "turboQuant", 6, 8, 128, 4, 2, 3000, 0),
 ]
 
 

@@ -68,13 +68,16 @@ def test_vector_keys(q, method, kb, vb, d, nq, kv, tokens):
 
 
 @pytest.mark.parametrize("tokens", TOKENS)
-@pytest.mark.parametrize("kb,vb,d,nq,kv,group", [(4, 3, 128, 4, 2, 64), (2, 2, 64, 8, 1, 128), (3, 4, 128, 6, 1, 64),
-                                                 (3, 3, 64, 2, 3, 64)])
-def test_channel_keys(q, kb, vb, d, nq, kv, group, tokens):
-    """Head-major per-channel keys with uneven channels, and a partial last group."""
+@pytest.mark.parametrize("method,kb,vb,d,nq,kv,group",
+                         [("turboQuant", 4, 3, 128, 4, 2, 64), ("turboQuant", 2, 2, 64, 8, 1, 128),
+                          ("turboQuant", 3, 4, 128, 6, 1, 64), ("turboQuant", 3, 3, 64, 2, 3, 64),
+                          ("polarQuant", 4, 4, 128, 4, 2, 64), ("polarQuant", 2, 4, 64, 8, 1, 64),
+                          ("polarQuant", 3, 2, 64, 1, 2, 128), ("polarQuant", 4, 3, 128, 6, 1, 128)])
+def test_channel_keys(q, method, kb, vb, d, nq, kv, group, tokens):
+    """Head-major per-channel keys with uneven channels, and a partial last group; values of either method."""
     import torch
     import pitch_amd as P
-    label = f"channel k{kb} v{vb} d={d} nq={nq} kv={kv} G={group} T={tokens}"
+    label = f"channel k{kb} {method} v{vb} d={d} nq={nq} kv={kv} G={group} T={tokens}"
     print(label, flush=True)
     rng = np.random.default_rng(tokens + d + nq + 7)
     stride = -(-tokens // group) * group
@@ -94,13 +97,96 @@ def test_channel_keys(q, kb, vb, d, nq, kv, group, tokens):
     dq, dkp, dkr, dvp, dvs = _dev(q, Q, kp, kr, vp, vs)
     out, lse = torch.empty(kv, nq, d, device=q.device), torch.empty(kv, nq, device=q.device)
     q.enqueueAttentionDecode(dq, dkp, dkr, dvp, dvs, out, tokens, P.ChannelQuantConfig(d, kb, group),
-                             P.QuantConfig("turboQuant", d, vb, 202), qPerKv=nq, kvHeads=kv, headStride=stride, lse=lse)
+                             P.QuantConfig(method, d, vb, 202), qPerKv=nq, kvHeads=kv, headStride=stride, lse=lse)
     out, lse = out.cpu().numpy().astype(np.float64), lse.cpu().numpy().astype(np.float64)
     for h in range(kv):
         Kd = O.channel_decode(kcodes[h], kr[h], kb, group).astype(np.float64)
-        Vd = O.turbo_decode(vc[h, :tokens], vs[h, :tokens].astype(np.float64), vb, 202)
+        Vd = O.DECODERS[method](vc[h, :tokens], vs[h, :tokens].astype(np.float64), vb, 202)
         ro, rl = O.attend(Q[h].astype(np.float64), Kd, Vd, 1 / math.sqrt(d))
         _compare(out[h], lse[h], ro, rl, f"{label} head {h}")
+
+
+# equal widths, whose keys and values share a table: lengths above those that attn_chunk serves
+EQUAL = [("turboQuant", 4, 128, 4, 8, 5000), ("polarQuant", 3, 128, 8, 8, 5001), ("turboQuant", 4, 128, 1, 8, 8193),
+         ("turboQuant", 2, 64, 2, 16, 9000), ("polarQuant", 4, 64, 8, 12, 12000), ("turboQuant", 3, 128, 3, 48, 1001)]
+
+
+@pytest.mark.parametrize("head_major", [False, True])
+@pytest.mark.parametrize("method,bits,d,nq,kv,tokens", EQUAL)
+def test_equal_widths(q, method, bits, d, nq, kv, tokens, head_major):
+    """Token-major caches put a chunk's heads on one XCD (8 chunks per head and more) or leave four chunks per head (48
+    heads); head-major ones do neither. The first, a middle and the last head are compared."""
+    import torch
+    import pitch_amd as P
+    print(f"{method} b={bits} d={d} nq={nq} kv={kv} T={tokens} head-major={head_major}", flush=True)
+    rng = np.random.default_rng(tokens + d + nq)
+    kc, kp = _packed(rng, kv, tokens, d, bits)
+    vc, vp = _packed(rng, kv, tokens, d, bits)
+    ks = np.exp(rng.uniform(1.5, 3.0, (kv, tokens))).astype(np.float32)
+    vs = np.exp(rng.uniform(-1.0, 1.0, (kv, tokens))).astype(np.float32)
+    Q = rng.standard_normal((kv, nq, d)).astype(np.float32)
+    order = (0, 1) if head_major else (1, 0)
+    dq, dkc, dvc = _dev(q, Q, kp.transpose(*order, 2), vp.transpose(*order, 2))
+    dks, dvs = _dev(q, ks.transpose(order), vs.transpose(order))
+    out, lse = torch.empty(kv, nq, d, device=q.device), torch.empty(kv, nq, device=q.device)
+    layout = dict(headStride=tokens) if head_major else dict(tokenStride=kv, headStride=1)
+    q.enqueueAttentionDecode(dq, dkc, dks, dvc, dvs, out, tokens, P.QuantConfig(method, d, bits, 101),
+                             P.QuantConfig(method, d, bits, 202), qPerKv=nq, kvHeads=kv, lse=lse, **layout)
+    out, lse = out.cpu().numpy().astype(np.float64), lse.cpu().numpy().astype(np.float64)
+    for h in (0, kv // 2, kv - 1):
+        ro, rl = O.attention_decode(Q[h].astype(np.float64), kc[h], ks[h], vc[h], vs[h], method, bits, method, bits,
+                                    1 / math.sqrt(d), 101, 202)
+        _compare(out[h], lse[h], ro, rl, f"head {h}")
+
+
+@pytest.mark.parametrize("nq", [4, 8])
+@pytest.mark.parametrize("keys", ["equal", "unequal", "bias", "channel"])
+def test_late_maxima(q, keys, nq):
+    """Scores up to 40 and more whose size grows with the position, so that the maximum of every wave's second and later
+    tiles is above that of the tiles before and its accumulators are rescaled: 24 KV heads of 250 tiles, 8 workgroups per
+    head, two tiles per wave (four to six with eight queries or the key-bias term)."""
+    import torch
+    import pitch_amd as P
+    print(keys, nq, flush=True)
+    kv, tokens, d, vb, group = 24, 16000, 64, 4 if keys == "equal" else 3, 64
+    rng = np.random.default_rng(nq)
+    ramp = np.linspace(0.2, 1.0, tokens)
+    vc, vp = _packed(rng, kv, tokens, d, vb)
+    vs = np.exp(rng.uniform(-1.0, 1.0, (kv, tokens))).astype(np.float32)
+    Q = rng.standard_normal((kv, nq, d)).astype(np.float32)
+    more, heads = {}, (0, kv - 1)
+    if keys == "channel":
+        K = rng.standard_normal((kv, tokens, d)).astype(np.float32) * (10 * ramp[:, None]).astype(np.float32)
+        enc = [O.channel_encode(K[h], 4, group) for h in range(kv)]
+        kp = np.stack([np.frombuffer(O.pack_codes(c, 4), np.uint8).reshape(tokens, -1) for c, _ in enc])
+        ks = np.stack([r for _, r in enc])
+        kcfg = P.ChannelQuantConfig(d, 4, group)
+        Kd = {h: O.channel_decode(*enc[h], 4, group).astype(np.float64) for h in heads}
+    else:
+        kc, kp = _packed(rng, kv, tokens, d, 4)
+        ks = (80 * ramp * np.ones((kv, 1))).astype(np.float32)
+        kcfg = P.QuantConfig("turboQuant", d, 4, 101)
+        Kd = {h: O.turbo_decode(kc[h], ks[h].astype(np.float64), 4, 101) for h in heads}
+        if keys == "bias":
+            ang = np.arange(tokens)[:, None] * (1e4 ** -(np.arange(d // 2) / (d // 2)))[None]
+            cos, sin = (np.concatenate([f(ang)] * 2, 1).astype(np.float32) for f in (np.cos, np.sin))
+            b = rng.standard_normal((kv, d)).astype(np.float32)
+            more["keyBias"] = P.KeyBias(*_dev(q, b, cos, sin), firstPosition=0, heads=kv)
+            kp, ks, vp = kp.transpose(1, 0, 2), ks.T, vp.transpose(1, 0, 2)
+            more.update(tokenStride=kv, headStride=1)
+            for h in heads:
+                half = np.concatenate([-b[h, d // 2:], b[h, :d // 2]])
+                Kd[h] = Kd[h] + b[h].astype(np.float64) * cos + half.astype(np.float64) * sin
+    dq, dkc, dks, dvc, dvs = _dev(q, Q, kp, ks, vp, vs.T if keys == "bias" else vs)
+    out, lse = torch.empty(kv, nq, d, device=q.device), torch.empty(kv, nq, device=q.device)
+    q.enqueueAttentionDecode(dq, dkc, dks, dvc, dvs, out, tokens, kcfg, P.QuantConfig("turboQuant", d, vb, 202),
+                             qPerKv=nq, kvHeads=kv, lse=lse, **(more or dict(headStride=tokens)))
+    out, lse = out.cpu().numpy().astype(np.float64), lse.cpu().numpy().astype(np.float64)
+    for h in heads:
+        Vd = O.turbo_decode(vc[h], vs[h].astype(np.float64), vb, 202)
+        ro, rl = O.attend(Q[h].astype(np.float64), Kd[h], Vd, 1 / math.sqrt(d))
+        assert rl.max() > 30, rl
+        _compare(out[h], lse[h], ro, rl, f"{keys} head {h}", 1e-4)
 
 
 @pytest.mark.parametrize("tokens", [1, 64, 65, 257, 4097])
