@@ -13,9 +13,12 @@
 //   * the other operand (rotated queries, softmax weights) is split too, its parts on rows that the few query heads
 //     of a KV head leave empty: row 4 part + head for up to four heads (three parts of the query, two of the
 //     weights), row 8 part + head for up to eight (two parts). The parts' products are summed in float32.
-// Two float16 parts hold a table value to 2^-23, three a query to 2^-33. Error against float64 (relative L2, mean of
-// ten seeds), attn_chunk's -> this kernel's: 8 KV x 4 queries, 16000 tokens 6.9e-7 -> 4.9e-7; key-bias term, 2 KV x 6,
-// 2000 tokens 1.1e-6 -> 7.0e-7; per-channel keys 0.6 - 1.8e-6 -> 2.7 - 8.5e-7.
+// Two float16 parts hold a table value, a cos or sin value or (five to eight heads) a query to 2^-23, three a query to
+// 2^-33; a weight is held to 2^-22 down to 2^-28 of the largest of its tile. Error against float64 (relative L2, mean over
+// 4 seeds x 2 methods x 4 width pairs x 700, 5000 and 40000 tokens), the float32 kernels' -> these: d = 128, up to four
+// heads 9.4e-7 -> 6.6e-7, five to eight 7.8e-7 -> 6.5e-7; d = 64 7.5e-7 -> 6.5e-7, 6.6e-7 -> 6.2e-7; key-bias term, d =
+// 128 1.29e-6 -> 9.1e-7, 1.25e-6 -> 8.8e-7; per-channel keys (40 seeds each), d = 128, four heads 1.2 - 1.7e-6 -> 5.1 -
+// 7.7e-7, eight 1.3 - 1.8e-6 -> 0.8 - 1.0e-6. Single calls scatter by a factor of three around these, either way.
 // Per-channel keys need no table: a code is exact in bfloat16, so a group's query products q_j step_j are split into
 // three bfloat16 parts (24 bits) and the codes are converted in registers (v_mfma_f32_16x16x32_bf16).
 //
@@ -23,13 +26,15 @@
 // separates the phases and the waves of a SIMD hide each other's loads; a workgroup's waves merge through LDS at the
 // end and attn_combine merges the workgroups. Weighted values are added up per tile, scores of table keys per two steps,
 // in float32 on the VALU: the matrix cores truncate what they align to a running sum, which a long chain would feel
-// (one chain per score: mean 6.3e-7 and at most 1.35e-6 of ten seeds, pairs of steps 4.9e-7 and 6.2e-7; same time).
+// (one chain per score: mean 6.3e-7 and at most 1.35e-6 of ten seeds, pairs of steps 4.9e-7 and 6.2e-7; same time). Scores
+// of per-channel keys are one chain of d / 32 steps, twice as many for five to eight heads: starting each step from zero
+// changes nothing for four heads (per-head mean 3.26e-7 and 3.24e-7 at d = 128) and takes eight from 4.2e-7 to 3.4e-7.
 //
-// Bound: long calls by their reads (Llama-3-8B layer, 8 KV x 4 queries, b = 4, token-major: 131072 tokens 64 -> 43 us,
-// 3.3 TB/s; with every tile read from the same few, so out of L2, 8 us less, without the loads 16 less), the rest by
-// fixed latency: launch, tables, one tile and the second launch are 10 - 12 us. Same layer: 16000 tokens 23.2 -> 13.7,
-// 32768 tokens 23.0 -> 17.6; per-channel keys of four bits and values of three, 131072 tokens 72.8 -> 42; key-bias
-// term, 2 KV x 6, 2000 tokens 21.8 -> 18.5, 4 KV x 4, 48606 tokens 210 -> 35.
+// Bound: long calls by their reads (Llama-3-8B layer, 8 KV x 4 queries, b = 4, token-major, us per call in a graph with
+// the float32 kernels -> here: 131072 tokens 64.7 -> 46.5, 3.0 TB/s; with every tile read from the same few, so out of
+// L2, 8 less, without the loads 16 less), the rest by fixed latency: launch, tables, one tile and the second launch are
+// 10 - 12 us. Same layer: 16000 tokens 23.4 -> 14.2, 32768 tokens 23.4 -> 18.6; per-channel keys of four bits and values of
+// three, 131072 tokens 73.5 -> 44.7; key-bias term, 2 KV x 6, 2000 tokens 21.2 -> 17.8, 4 KV x 4, 48606 tokens 203 -> 36.
 #include "pitch_attn_shared.h"
 
 #ifndef PITCH_DIM
@@ -250,8 +255,8 @@ constexpr bool kBias = PITCH_KIND == kAttnKindTurboBias || PITCH_KIND == kAttnKi
 constexpr bool kKeyPolar = PITCH_KIND == kAttnKindPolar || PITCH_KIND == kAttnKindPolarBias;
 constexpr bool kValPolar = kKeyPolar || PITCH_KIND == kAttnKindChanPolar;
 
-// Waves of a workgroup, one workgroup per compute unit: three per SIMD (168 registers each) for up to four heads, two
-// (256) for eight and with the key-bias term, whose accumulators would spill.
+// Most waves of a workgroup, one workgroup per compute unit: four per SIMD (128 registers each) for up to four heads, two
+// (256) for five to eight and with the key-bias term, whose accumulators would spill.
 constexpr uint32_t max_waves(bool q8) { return q8 || kBias ? 8 : kAttnCodesWaves; }
 
 template <int D, int KB, int VB, bool Q8>
@@ -837,7 +842,7 @@ __global__ __launch_bounds__(64 * max_waves(Q8)) void attn_codes(AttnArgs a) {
   }
   __syncthreads();
   float* const s_out = (float*)s_q;  // heads x D: the query operand's space, no longer read
-  static_assert(S::kQ >= NH * D || NH * D <= S::kTabK + S::kTabV + S::kQ, "merged heads fit");
+  static_assert(S::kQ >= NH * D, "merged heads fit the query operand's space");
   const int nqh = (int)a.nq;
   for (int x = tid; x < nqh * D; x += blockDim.x) {
     const int h = x / D, j = x % D;
