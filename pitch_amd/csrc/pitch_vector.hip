@@ -2387,8 +2387,9 @@ constexpr EncKind enc_kind() {
   return EncKind::kTeam;
 }
 // Whether a call of so many vectors runs the LDS-transposed encoder where enc_kind names it; the others run the team
-// encoder, with the same bytes. Both sides below are us per call, team and transposed, d = 256, bfloat16 (float16, d = 512
-// and 1024 alike). 16-bit TurboQuant takes it from 2^23 coordinates: below two of its resident rounds (2 waves per SIMD
+// encoder, with the same bytes (TurboQuant of eight bits: but for 2 codes in 10^9 that lie within 2^-36 of an edge, which
+// the bucket table rounds). Both sides below are us per call, team and transposed, d = 256, bfloat16 (float16, d = 512 and
+// 1024 alike). 16-bit TurboQuant takes it from 2^23 coordinates: below two of its resident rounds (2 waves per SIMD
 // against the team encoder's 4) its fixed cost loses (64 vectors, b = 2: 4.4 and 5.2; 16744, b = 4: 7.7 and 9.3; 40000, b =
 // 8: 13.8 and 13.5; 131072, b = 3: 41.0 and 31.8). PolarQuant of 2 - 5 bits gains at every size (64 vectors, b = 2: 6.7
 // and 5.8, b = 5: 6.6 and 6.3; 4096, b = 5: 8.7 and 7.3; 131072, b = 3: 68.8 and 35.1). Its octant table grows with 2^b, so
