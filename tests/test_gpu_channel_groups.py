@@ -89,3 +89,26 @@ def test_rows_of_small_groups(q, dim, bits, group, tokens):
     q.enqueuePerChannelEncode(torch.from_numpy(x).to(q.device), c, r, tokens, cfg)
     assert c.cpu().numpy().tobytes() == O.pack_codes(codes, bits)
     assert np.array_equal(r.cpu().numpy().view(np.uint16), ranges.reshape(-1).view(np.uint16))
+
+
+@pytest.mark.parametrize("io", ["float32", "bfloat16"])
+@pytest.mark.parametrize("rows", [1, 31, 32, 33, 64, 65, 127])
+@pytest.mark.parametrize("dim,bits,group", [(64, 4, 128), (80, 3, 128), (128, 8, 100), (28, 5, 65), (128, 2, 64)])
+def test_appends_to_a_short_last_group(q, dim, bits, group, rows, io):
+    """Appends of single tokens to the last of two groups: what is written equals one encode of all tokens, for every count
+    of rows that the last group can have, and the first group stays."""
+    import torch
+    rows = min(rows, group)
+    print(f"d={dim} b={bits} G={group} rows={rows} {io}", flush=True)
+    tokens = group + rows
+    x = np.random.default_rng(dim + rows).standard_normal((tokens, dim)).astype(np.float32)
+    t = torch.from_numpy(x).to(getattr(torch, io))
+    codes, ranges = O.channel_encode(t.float().numpy(), bits, group)
+    cfg = q.channelConfig(dim, bits, group)
+    dev = t.to(q.device)
+    c = torch.zeros(tokens * cfg.codeStride, dtype=torch.uint8, device=q.device)
+    r = torch.zeros(ranges.size, dtype=torch.int16, device=q.device)
+    q.enqueuePerChannelEncode(dev, c, r, tokens - 1, cfg)
+    q.enqueuePerChannelAppend(dev, c, r, tokens, 1, cfg)
+    assert c.cpu().numpy().tobytes() == O.pack_codes(codes, bits)
+    assert np.array_equal(r.cpu().numpy().view(np.uint16), ranges.reshape(-1).view(np.uint16))
